@@ -192,12 +192,14 @@ int li_block_mask(int dtype, int32_t B, int32_t NH, int32_t D,
  * Built for block_size in {64, 128} and D in {64, 128}.
  *
  * workspace (optional, device, 16-byte aligned, NULL allowed): scratch of
- * li_bsa_fwd_workspace_size() bytes.  With it, when the query tiles fill the
- * device's CUs unevenly, the tiles of the last partial round are each split
- * into two halves of their block list that run on different CUs and are
- * combined by a second kernel on the same stream.  Without it (or when it is
- * smaller than required) every tile runs whole.  Results are the same up to
- * fp32 rounding of the combination.
+ * li_bsa_fwd_workspace_size_cols() bytes.  With it, when the query tiles fill
+ * the device's CUs unevenly, the tiles of the last partial round are each
+ * split into pieces of their block list that run on different CUs and are
+ * combined by a second kernel on the same stream.  A smaller workspace gets
+ * the best split that fits it (li_bsa_fwd_workspace_size() bytes hold two
+ * pieces of each tile of a last round at most half full); without one every
+ * tile runs whole.  Results are the same up to fp32 rounding of the
+ * combination.
  *
  * flags: a combination of
  *  LI_BSA_BALANCE for rows of unequal length (ragged budgets): with the
@@ -262,8 +264,8 @@ int li_bsa_fwd_gather(int dtype, int32_t B, int32_t NH, int32_t D,
  * to a scratch array of li_bsa_fwd_noalloc_scratch_bytes() bytes (32 MiB)
  * that the library holds on each device it runs on until the process ends.
  * Same kernels, same split and order decisions and same results, bit for
- * bit, as li_bsa_fwd_gather given a workspace of li_bsa_fwd_workspace_size()
- * bytes.  LI_ERR_TOO_LARGE when that workspace would exceed the scratch.
+ * bit, as li_bsa_fwd_gather given a workspace of
+ * li_bsa_fwd_workspace_size_cols() bytes.  LI_ERR_TOO_LARGE when that workspace would exceed the scratch.
  * Every call on a device shares that device's scratch: calls that overlap
  * on one GPU (other streams, other threads) race and must be serialised by
  * the caller.  No counterpart in the reference: for callers that cannot
@@ -285,12 +287,20 @@ int64_t li_bsa_fwd_noalloc_scratch_bytes(void);
 
 /*
  * Workspace bytes li_bsa_fwd / li_bsa_fwd_gather can use for these sizes on
- * the current device: room for the tail split's partials or for the tile
- * order of LI_BSA_BALANCE, whichever is larger (0 for D != 128).  Depends on
- * the device's CU count.  No counterpart in the reference (its Triton launch
- * has neither).
+ * the current device, without the width of the lists: room for two pieces of
+ * each tile of a last round that is at most half full or for the tile order
+ * of LI_BSA_BALANCE, whichever is larger (0 for D != 128).  Depends on the
+ * device's CU count.  No counterpart in the reference (its Triton launch has
+ * neither).
  */
 int64_t li_bsa_fwd_workspace_size(int32_t B, int32_t NH, int32_t Lq, int32_t D, int32_t block_size);
+/*
+ * The same for lists of n_cols columns (dense calls: their number of key
+ * blocks): room for the split that these sizes get, at most 32 MiB of
+ * partials, or for the tile order.
+ */
+int64_t li_bsa_fwd_workspace_size_cols(int32_t B, int32_t NH, int32_t Lq, int32_t D, int32_t block_size,
+                                       int32_t n_cols);
 
 /*
  * Dense attention over all keys: the reference's dense fallback

@@ -54,17 +54,18 @@ struct BsaArgs {
   float qk_scale;
   // Query tiles of the launch (B * NH * nqt), placed on the XCDs by unit_tile.
   int32_t ntiles;
-  // Tail split (D = 128, BS = 128 kernel only; ntiles a multiple of 8): XCD x
-  // (unit ids x, x + 8, ...) owns the xtiles = ntiles / 8 tiles from
-  // x * xtiles on.  When xsplit > 0, the last xsplit of them run as two
-  // halves of their kept-block list, the first ceil(count / 2) blocks and
-  // the rest.  Slot s of XCD x (unit 8 s + x) runs whole tile x * xtiles + s
-  // for s < xtiles - xsplit, then come the first halves of the split tiles,
-  // then their second halves, so a split tile's halves stay on the XCD whose
-  // L2 holds its head's keys.  Half e of split tile j of XCD x writes
-  // unnormalised fp32 O and (m, l) rows to partial slot 2 (x * xsplit + j) +
-  // e of `part` for the merge kernel.
-  int32_t xtiles, xsplit;
+  // Split (D = 128, BS = 128 kernel only): XCD x (unit ids x, x + 8, ...) owns
+  // a contiguous range of tiles (xcd_first_tile, xcd_tiles).  When xparts > 0,
+  // the first xwhole of them run whole and the others, at most xsplit, as
+  // xparts pieces of their kept-block list each (the first count % xparts
+  // pieces one entry longer).  Slots s < xwhole of XCD x (unit 8 s + x) run its
+  // whole tiles; slot xwhole + e xsplit + j runs piece e of its split tile j,
+  // so a tile's pieces stay on the XCD whose L2 holds its head's keys (an XCD
+  // with one split tile fewer leaves j = xsplit - 1 idle).  The piece writes
+  // unnormalised fp32 O and (m, l) rows to partial slot (x xsplit + j) xparts
+  // + e of `part` for the merge kernel.
+  int32_t xwhole, xsplit, xparts;
+  uint32_t mg_split, mg_parts;  // udiv16 magics of xsplit and xparts
   float* part;
   // Optional dispatch order of the tiles (a permutation of [0, ntiles);
   // never with the tail split): position p of the XCD-aware unit order runs
@@ -90,6 +91,14 @@ struct BsaArgs {
   int32_t gen_pairs;
 };
 
+// The contiguous tiles of one XCD: the tiles dealt in ranges of ntiles / 8, the
+// first ntiles % 8 ranges one longer.
+__device__ __forceinline__ int xcd_first_tile(const BsaArgs& a, int x) {
+  const int per = a.ntiles >> 3, rem = a.ntiles & 7;
+  return x * per + (x < rem ? x : rem);
+}
+__device__ __forceinline__ int xcd_tiles(const BsaArgs& a, int x) { return (a.ntiles >> 3) + (x < (a.ntiles & 7) ? 1 : 0); }
+
 // Tile of work unit `id` (< a.ntiles): ids are dealt round-robin over
 // the 8 XCDs, so they are remapped to give each XCD a contiguous range of
 // positions; a.order, when given, names the tile at each position.
@@ -100,8 +109,7 @@ __device__ __forceinline__ int unit_tile(const BsaArgs& a, int id) {
     const int c = a.xchunk;
     pos = ((slot / c) * 8 + xcd) * c + slot % c;
   } else {
-    const int per = a.ntiles >> 3, rem = a.ntiles & 7;
-    pos = xcd * per + (xcd < rem ? xcd : rem) + slot;
+    pos = xcd_first_tile(a, xcd) + slot;
   }
   if (!a.order) return pos;
   const int t = __builtin_amdgcn_readfirstlane(a.order[pos]);

@@ -454,20 +454,20 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   const int l32 = lane & 31, hl = lane >> 5;
 
   // Work unit -> query tile: unit_tile gives each XCD (ids are dealt
-  // round-robin over the 8 XCDs) a contiguous range of tiles; with the tail
-  // split, the last slots of an XCD run the halves of its split tiles
-  // (`half` = which half, `pslot` = its partial slot).
+  // round-robin over the 8 XCDs) a contiguous range of tiles; with the
+  // split, the last slots of an XCD run the pieces of its split tiles
+  // (`piece` = which one, `pslot` = its partial slot).
   const int id = blockIdx.x;
-  int tile, half = -1, pslot = 0;
-  if (a.xsplit == 0 || (id >> 3) < a.xtiles - a.xsplit) {
+  int tile, piece = 0, pslot = -1;
+  if (a.xparts == 0 || (id >> 3) < a.xwhole) {
     tile = unit_tile(a, id);
   } else {
-    const int x = id & 7;
-    int j = (id >> 3) - (a.xtiles - a.xsplit);
-    half = j >= a.xsplit ? 1 : 0;
-    j -= half ? a.xsplit : 0;
-    tile = x * a.xtiles + (a.xtiles - a.xsplit) + j;
-    pslot = 2 * (x * a.xsplit + j) + half;
+    const int x = id & 7, p = (id >> 3) - a.xwhole;
+    piece = (int)udiv16(p, a.mg_split);
+    const int j = p - piece * a.xsplit;
+    if (j >= xcd_tiles(a, x) - a.xwhole) return;  // the whole workgroup, before any barrier
+    tile = xcd_first_tile(a, x) + a.xwhole + j;
+    pslot = (x * a.xsplit + j) * a.xparts + piece;
   }
   const int bh = tile / a.nqt, m = tile % a.nqt;
   const int b = bh / a.NH, h = bh % a.NH;
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   const int32_t* irow = DN ? nullptr : a.idx + b * a.is[0] + h * a.is[1] + (int64_t)m * a.is[2];
   // The first four entries of the row (clamped to its columns), read through
   // the scalar cache without waiting for the count, which picks among them;
-  // the second half of a split tile reads its own after the count.
+  // the later pieces of a split tile read their own after the count.
   int r0 = -1, r1 = -1, r2 = -1, r3 = -1;
   auto read_first = [&](const int32_t* row, int ncols) LI_INLINE {
     const const_i32* rs = (const const_i32*)row;
@@ -535,29 +535,25 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
     r2 = rs[(int64_t)(2 < ncols ? 2 : ncols - 1) * is3];
     r3 = rs[(int64_t)(3 < ncols ? 3 : ncols - 1) * is3];
   };
-  if (!DN && half != 1 && a.n_cols > 0) read_first(irow, a.n_cols);
+  if (!DN && piece == 0 && a.n_cols > 0) read_first(irow, a.n_cols);
   const int32_t* cnt_at = DN ? nullptr : a.cnt + b * a.cs[0] + h * a.cs[1] + (int64_t)m * a.cs[2];
   int count = DN ? a.n_cols : *cnt_at;
   count = count < 0 ? 0 : (count > a.n_cols ? a.n_cols : count);
   count = __builtin_amdgcn_readfirstlane(count);
   int id_base = 0;
-  if (half >= 0) {
-    const int h0 = (count + 1) >> 1;
-    if constexpr (!DN) irow += half ? (int64_t)h0 * a.is[3] : 0;
-    id_base = half ? h0 : 0;
-    count = half ? count - h0 : h0;
-    if (!DN && half == 1 && a.n_cols - h0 > 0) read_first(irow, a.n_cols - h0);
+  if (pslot >= 0) {
+    const int base = (int)udiv16(count, a.mg_parts), longer = count - base * a.xparts;
+    id_base = piece * base + (piece < longer ? piece : longer);
+    count = base + (piece < longer ? 1 : 0);
+    if constexpr (!DN) irow += (int64_t)id_base * a.is[3];
+    if (!DN && piece > 0 && a.n_cols - id_base > 0) read_first(irow, a.n_cols - id_base);
   }
-  // An empty list (or an empty half of a split tile) runs as one block with
+  // An empty list (or an empty piece of a split tile) runs as one block with
   // an out-of-range id, which gets all-zero probabilities: the epilogue then
   // writes zero rows and an LSE of -inf (zero partials and (m, l) = (-inf, 0)
-  // for a half), with no early exit to hold back the loads above.
+  // for a piece), with no early exit to hold back the loads above.
   const bool empty = count == 0;
   count = empty ? 1 : count;
-  // Partial rows of a split unit: O as [128 rows][128 d] fp32, then (m, l).
-  float* part_o = half >= 0 ? a.part + (int64_t)pslot * BS * (D + 2) : nullptr;
-  float* part_ml = half >= 0 ? part_o + BS * D : nullptr;
-
   // Output row of tile row rt, or null when it is not stored (past Lq, or
   // outside the token grid on the fused path).
   auto out_row = [&](int rt) LI_INLINE -> uint16_t* {
@@ -1042,7 +1038,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
     // (the same clamp as block_id), so a read costs no index arithmetic.
     const int64_t ist = a.is[3];
     // An empty unit's row may have no entry to read (no columns, or the
-    // second half of a one-block list): its pointer is the count it was
+    // later pieces of a short list): its pointer is the count it was
     // given, which is readable, and the value read is never used.
     const_i32* idp = DN ? nullptr
                         : empty ? (const_i32*)cnt_at
@@ -1241,7 +1237,10 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
     const float a1 = none ? 0.0f : __builtin_amdgcn_exp2f(m1 - mm);
     const float l = lrow * a0 + l1 * a1;
     const int rt = 32 * qq + l32;
-    if (half >= 0) {
+    if (pslot >= 0) {
+      // Partial rows of a piece: O as [128 rows][128 d] fp32, then (m, l).
+      float* part_o = a.part + (int64_t)pslot * BS * (D + 2);
+      float* part_ml = part_o + BS * D;
       float* prow = part_o + rt * D;
 #pragma unroll
       for (int dt = 0; dt < C::NDT; ++dt)
@@ -1280,115 +1279,140 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   }
 }
 
-// Combines the two halves of each split query tile: O = (O0 a0 + O1 a1) /
-// (l0 a0 + l1 a1) with a_i = 2^(m_i - max(m0, m1)); lse = max + log2(l).  Four
-// workgroups per split tile (32 rows each), eight threads per row (16 d each,
-// 64 contiguous bytes of each partial).  Split tile p = x * xsplit + j is
-// tile j of the split tiles of XCD x.
-template <typename E, bool G = false>
+// Combines the pieces of each split query tile: O = sum_e O_e a_e / sum_e l_e
+// a_e with a_e = 2^(m_e - max_e m_e); lse = max + log2(sum).  Bound by the
+// latency of the partials' loads (65 KiB a piece), so they are taken NB pieces
+// at a time, O with (m, l), before any of them is used, and the running sums
+// are rescaled once per NB (2 for two pieces, else 4).  Eight workgroups per split tile (16 rows
+// each), 16 threads per row (8 d each, 512 contiguous bytes of a partial per
+// row).  Workgroups past the last split tile of an XCD, whose range is one tile
+// shorter than the longest, do nothing.
+template <typename E, bool G, int NB>
 __global__ __launch_bounds__(256) void bsa_merge_kernel(BsaArgs a) {
   constexpr int BS = 128, D = 128;
-  const int p = blockIdx.x >> 2;
+  const int p = blockIdx.x >> 3;
   const int x = p / a.xsplit, j = p - x * a.xsplit;
-  const int tile = x * a.xtiles + (a.xtiles - a.xsplit) + j;
+  if (j >= xcd_tiles(a, x) - a.xwhole) return;
+  const int tile = xcd_first_tile(a, x) + a.xwhole + j;
   const int bh = tile / a.nqt, m = tile % a.nqt;
-  const int rt = (blockIdx.x & 3) * 32 + (threadIdx.x >> 3), dq = threadIdx.x & 7;
+  const int rt = (blockIdx.x & 7) * 16 + (threadIdx.x >> 4), dq = threadIdx.x & 15;
   const int r = m * BS + rt;
   if (r >= a.Lq) return;
+  constexpr int64_t PS = BS * (D + 2);
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  const float* p0 = a.part + (int64_t)p * a.xparts * PS;
+  const float* o0 = p0 + rt * D + 8 * dq;
+  const float* ml0 = p0 + BS * D + 2 * rt;
+  float mm = -__builtin_inff(), l = 0.0f;
+  float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  for (int e0 = 0; e0 < a.xparts; e0 += NB) {
+    f32x4 o[NB][2];
+    f32x2 ml[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      // Past the last piece: its rows again, with weight 0.
+      const int64_t at = (e0 + i < a.xparts ? e0 + i : a.xparts - 1) * PS;
+      ml[i] = *reinterpret_cast<const f32x2*>(ml0 + at);
+      o[i][0] = *reinterpret_cast<const f32x4*>(o0 + at);
+      o[i][1] = *reinterpret_cast<const f32x4*>(o0 + at + 4);
+    }
+    float mx = mm;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) mx = __builtin_fmaxf(mx, ml[i][0]);
+    if (mx == -__builtin_inff()) continue;  // nothing kept so far
+    const float keep = __builtin_amdgcn_exp2f(mm - mx);
+    mm = mx;
+    l *= keep;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[d] *= keep;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const float w = e0 + i < a.xparts ? __builtin_amdgcn_exp2f(ml[i][0] - mx) : 0.0f;
+      l += ml[i][1] * w;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) acc[d] += o[i][d >> 2][d & 3] * w;
+    }
+  }
   // Padding rows of the grid have no output token but do have an LSE.
   uint16_t* orow = nullptr;
   if constexpr (G) {
     const int b = bh / a.NH, h = bh % a.NH;
     bool ok;
-    const int32_t l = tile_token(a.g, a.g.Tq, m, rt, ok);
-    if (ok && l < a.g.q_tokens) orow = a.out + b * a.g.os[0] + h * a.g.os[1] + (int64_t)l * a.g.os[2] + 16 * dq;
+    const int32_t t = tile_token(a.g, a.g.Tq, m, rt, ok);
+    if (ok && t < a.g.q_tokens) orow = a.out + b * a.g.os[0] + h * a.g.os[1] + (int64_t)t * a.g.os[2] + 8 * dq;
   } else {
-    orow = a.out + ((int64_t)bh * a.Lq + r) * D + 16 * dq;
+    orow = a.out + ((int64_t)bh * a.Lq + r) * D + 8 * dq;
   }
-  const float* p0 = a.part + (int64_t)(2 * p) * BS * (D + 2);
-  const float* p1 = p0 + BS * (D + 2);
-  const float m0 = p0[BS * D + 2 * rt], l0 = p0[BS * D + 2 * rt + 1];
-  const float m1 = p1[BS * D + 2 * rt], l1 = p1[BS * D + 2 * rt + 1];
-  const float mm = __builtin_fmaxf(m0, m1);
-  const bool none = mm == -__builtin_inff();
-  const float a0 = none ? 0.0f : __builtin_amdgcn_exp2f(m0 - mm);
-  const float a1 = none ? 0.0f : __builtin_amdgcn_exp2f(m1 - mm);
-  const float l = l0 * a0 + l1 * a1;
   if (orow) {
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const f32x4* o0 = reinterpret_cast<const f32x4*>(p0 + rt * D + 16 * dq);
-    const f32x4* o1 = reinterpret_cast<const f32x4*>(p1 + rt * D + 16 * dq);
-    f32x4 x0[4], x1[4];
+    u32x4 pk;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x0[i] = o0[i];
-      x1[i] = o1[i];
-    }
-    u32x4 pk[2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      pk[i >> 1][2 * (i & 1)] = cvt_pk<E>((x0[i][0] * a0 + x1[i][0] * a1) * inv, (x0[i][1] * a0 + x1[i][1] * a1) * inv);
-      pk[i >> 1][2 * (i & 1) + 1] =
-          cvt_pk<E>((x0[i][2] * a0 + x1[i][2] * a1) * inv, (x0[i][3] * a0 + x1[i][3] * a1) * inv);
-    }
-    *reinterpret_cast<u32x4*>(orow) = pk[0];
-    *reinterpret_cast<u32x4*>(orow + 8) = pk[1];
+    for (int i = 0; i < 4; ++i) pk[i] = cvt_pk<E>(acc[2 * i] * inv, acc[2 * i + 1] * inv);
+    *reinterpret_cast<u32x4*>(orow) = pk;
   }
-  if (a.lse && dq == 0) a.lse[(int64_t)bh * a.Lq + r] = none ? -__builtin_inff() : mm + __builtin_log2f(l);
+  if (a.lse && dq == 0) a.lse[(int64_t)bh * a.Lq + r] = mm == -__builtin_inff() ? mm : mm + __builtin_log2f(l);
+}
+
+// Workgroups of an attention launch: the tiles, or per XCD its whole tiles and
+// the pieces of at most xsplit split ones.
+int attn_units(const BsaArgs& a) { return a.xparts == 0 ? a.ntiles : 8 * (a.xwhole + a.xsplit * a.xparts); }
+
+template <typename E, bool G>
+void launch_merge(const BsaArgs& a, hipStream_t s) {
+  const dim3 grid(8 * 8 * a.xsplit);
+  if (a.xparts == 2)
+    hipLaunchKernelGGL((bsa_merge_kernel<E, G, 2>), grid, dim3(256), 0, s, a);
+  else if (a.xparts > 2)
+    hipLaunchKernelGGL((bsa_merge_kernel<E, G, 4>), grid, dim3(256), 0, s, a);
 }
 
 template <typename E, bool DN = false>
-int launch_bsa_gather(BsaArgs& a, int tiles, hipStream_t s) {
-  const int nsplit = 8 * a.xsplit;
+int launch_bsa_gather(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
   if (a.zero_region)
-    hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, 128, true, false, DN, true>), dim3(tiles + nsplit),
+    hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, 128, true, false, DN, true>), dim3(attn_units(a)),
                        dim3(DmaCfg<128>::NTHR), 0, s, a);
   else
-    hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, 128, true, false, DN>), dim3(tiles + nsplit),
+    hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, 128, true, false, DN>), dim3(attn_units(a)),
                        dim3(DmaCfg<128>::NTHR), 0, s, a);
-  if (nsplit > 0) hipLaunchKernelGGL((bsa_merge_kernel<E, true>), dim3(4 * nsplit), dim3(256), 0, s, a);
+  launch_merge<E, true>(a, s);
   return launch_status();
 }
 
 template <bool G>
-int launch_bsa_fp8(BsaArgs& a, int tiles, hipStream_t s) {
-  const int nsplit = 8 * a.xsplit;
+int launch_bsa_fp8(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
   if (G && a.zero_region)
-    hipLaunchKernelGGL((bsa_fwd_dma_kernel<Bf16, 128, G, true, false, G>), dim3(tiles + nsplit),
+    hipLaunchKernelGGL((bsa_fwd_dma_kernel<Bf16, 128, G, true, false, G>), dim3(attn_units(a)),
                        dim3(DmaCfg<128>::NTHR), 0, s, a);
   else
-    hipLaunchKernelGGL((bsa_fwd_dma_kernel<Bf16, 128, G, true>), dim3(tiles + nsplit), dim3(DmaCfg<128>::NTHR),
+    hipLaunchKernelGGL((bsa_fwd_dma_kernel<Bf16, 128, G, true>), dim3(attn_units(a)), dim3(DmaCfg<128>::NTHR),
                        0, s, a);
-  if (nsplit > 0) hipLaunchKernelGGL((bsa_merge_kernel<Bf16, G>), dim3(4 * nsplit), dim3(256), 0, s, a);
+  launch_merge<Bf16, G>(a, s);
   return launch_status();
 }
 
 template <typename E, int BS>
-int launch_bsa_dma(BsaArgs& a, int tiles, hipStream_t s) {
-  const int nsplit = 8 * a.xsplit;
+int launch_bsa_dma(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
-  hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, BS>), dim3(tiles + nsplit), dim3(DmaCfg<BS>::NTHR), 0, s, a);
-  if constexpr (BS == 128) {
-    if (nsplit > 0) hipLaunchKernelGGL(bsa_merge_kernel<E>, dim3(4 * nsplit), dim3(256), 0, s, a);
-  }
+  hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, BS>), dim3(attn_units(a)), dim3(DmaCfg<BS>::NTHR), 0, s, a);
+  if constexpr (BS == 128) launch_merge<E, false>(a, s);
   return launch_status();
 }
 
 template <typename E, int BS, int D>
-int launch_bsa(BsaArgs& a, int tiles, hipStream_t s) {
+int launch_bsa(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
-  hipLaunchKernelGGL((bsa_fwd_kernel<E, BS, D>), dim3(tiles), dim3(Cfg<BS, D>::NTHR), 0, s, a);
+  hipLaunchKernelGGL((bsa_fwd_kernel<E, BS, D>), dim3(a.ntiles), dim3(Cfg<BS, D>::NTHR), 0, s, a);
   return launch_status();
 }
 
 template <typename E>
-int dispatch_bsa(BsaArgs& a, int bs, int D, int tiles, hipStream_t s) {
-  if (bs == 128 && D == 128) return launch_bsa_dma<E, 128>(a, tiles, s);
-  if (bs == 128 && D == 64) return launch_bsa<E, 128, 64>(a, tiles, s);
-  if (bs == 64 && D == 128) return launch_bsa_dma<E, 64>(a, tiles, s);
-  if (bs == 64 && D == 64) return launch_bsa<E, 64, 64>(a, tiles, s);
+int dispatch_bsa(BsaArgs& a, int bs, int D, hipStream_t s) {
+  if (bs == 128 && D == 128) return launch_bsa_dma<E, 128>(a, s);
+  if (bs == 128 && D == 64) return launch_bsa<E, 128, 64>(a, s);
+  if (bs == 64 && D == 128) return launch_bsa_dma<E, 64>(a, s);
+  if (bs == 64 && D == 64) return launch_bsa<E, 64, 64>(a, s);
   return LI_ERR_UNSUPPORTED;
 }
 
@@ -1455,33 +1479,65 @@ __global__ __launch_bounds__(1024) void bsa_order_kernel(BsaArgs a, int32_t* ord
   }
 }
 
-// Query tiles of each XCD whose block lists are split in halves.  The tiles
-// are dealt to the 8 XCDs in contiguous ranges of n = tiles / 8, and with
-// one 8-wave workgroup per CU an XCD of c = cus / 8 CUs runs its n tiles in
-// ceil(n / c) rounds, the last holding r = n % c tiles.  When r <= c / 2,
-// those r tiles run as 2 r halves on their own XCD (so that their key blocks
-// stay in its L2), and the last round is half as long (HY shape: 896 tiles,
-// n = 112, c = 32, r = 16).  A fuller last round is left whole: at the
-// Matrix-Game shape (n = 90, r = 26) uneven pieces (5/6 of a list on 26 CUs,
-// the 1/6 pieces on the other 6) ran as long as the whole round, each short
-// piece paying ~4 us of prologue and epilogue, and the merge added ~10 us.
-// No split when the tiles or the CUs do not divide evenly over the XCDs.
-int64_t split_per_xcd(int64_t tiles, int cus) {
-  if (cus <= 0 || cus % 8 != 0 || tiles % 8 != 0) return 0;
-  const int64_t n = tiles / 8, c = cus / 8;
-  if (n <= c) return 0;
-  const int64_t r = n % c;
-  return 2 * r <= c ? r : 0;
+// How the query tiles of one launch fill the CUs.  The tiles are dealt to the 8
+// XCDs in contiguous ranges of at most n = ceil(tiles / 8), and with one 8-wave
+// workgroup per CU an XCD of c = cus / 8 CUs runs its range in ceil(n / c)
+// rounds, the last holding r = n % c tiles (all of them when n < c).  Those r
+// tiles run as `parts` pieces of their block lists each when the pieces, in
+// ceil(r parts / c) rounds on the same XCD (so that their key blocks stay in
+// its L2), end sooner than whole tiles would.
+struct SplitPlan {
+  int32_t whole = 0, split = 0, parts = 0;  // whole and split tiles per XCD; parts = 0: no split
+};
+
+constexpr int64_t kPartBytes = 128 * (128 + 2) * 4;  // one piece: O and (m, l) of 128 rows
+// All pieces of a launch fit the scratch of the allocation-free entry point.
+constexpr int64_t kMaxPartBytes = 32ll << 20;
+
+// Time (us) of n units of `blocks` blocks each on c CUs: 9 us per unit (its
+// prologue, first softmax, epilogue and the CU's next dispatch) and 1.55 us per
+// block with every CU busy.  A block takes less when part of the chip idles,
+// down to 1.0 us at half of the CUs: the kernel runs at the card's power limit
+// (16 heads x 56 tiles x 51 blocks take 331 us on random data, 218 on zeros).
+double units_us(int64_t n, double blocks, int64_t c) {
+  constexpr double kUnit = 9.0, kBlock = 1.55, kBlockIdle = 1.0;
+  const double u = (double)(n % c) / (double)c;
+  const double last = u <= 0.5 ? kBlockIdle : kBlockIdle + (kBlock - kBlockIdle) * (u - 0.5) / 0.5;
+  return (double)(n / c) * (kUnit + blocks * kBlock) + (n % c ? kUnit + blocks * last : 0.0);
 }
 
-constexpr int64_t kPartBytesPerTile = 2 * 128 * (128 + 2) * 4;
+// The plan for lists of up to n_cols blocks within `bytes` of partials.  The
+// model's figures are within 10% of the measured ones at every size below
+// (attention and merge, us, bf16; heads x tiles x blocks):
+//   1 x  8 x 60: whole 67.2, 10 pieces 20.1   1 x 52 x 24: 31.6, 4 pieces 23.6
+//   1 x 52 x 72: 79.6, 4 pieces 40.0          2 x 52 x 40: 48.0, 2 pieces 41.9
+//   8 x 36 x 30: 92.8, 6 pieces 74.7          8 x 44 x 40: 118.9, 2 pieces 110.6
+//  16 x 49 x 50: 321.8, 8 pieces 284.7       16 x 56 x 51: 329.1, 2 pieces 325.2
+// and whole tiles stay the better ones at 3 x 52 x 72 (92.5 against 96.9), 2 x
+// 52 x 16 (24.0, 29.6), 1 x 52 x 8 (15.9, 18.5) and 8 x 58 x 39 (132.2, 145.4).
+SplitPlan plan_split(int64_t tiles, int64_t n_cols, int cus, int64_t bytes) {
+  constexpr double kMerge = 5.5, kMergePiece = 0.012;  // the merge launch, and its read of one piece
+  SplitPlan best;
+  if (cus <= 0 || cus % 8 != 0 || n_cols <= 0) return best;
+  const int64_t n = (tiles + 7) / 8, c = cus / 8, r = n % c;
+  if (r == 0) return best;
+  const int64_t most = (bytes < kMaxPartBytes ? bytes : kMaxPartBytes) / (8 * kPartBytes);  // pieces per XCD
+  double cost = units_us(r, (double)n_cols, c) - 1.0;  // a gain of less than 1 us is left
+  for (int64_t parts = 2; parts * r <= most && parts <= n_cols; ++parts) {
+    const double blocks = (double)((n_cols + parts - 1) / parts);
+    const double t = units_us(r * parts, blocks, c) + kMerge + kMergePiece * 8.0 * (double)(r * parts);
+    if (t < cost) {
+      cost = t;
+      best.whole = (int32_t)(n - r);
+      best.split = (int32_t)r;
+      best.parts = (int32_t)parts;
+    }
+  }
+  return best;
+}
 
 int64_t order_bytes(int64_t tiles) { return (tiles * 4 + 15) & ~(int64_t)15; }
 
-// Workspace use of one call: with LI_BSA_BALANCE (D = 128 kernels) the tile
-// order, built by bsa_order_kernel and no tail split; otherwise the tail
-// split's partials (D = 128, BS = 128).  Returns the launch status of the
-// order kernel (LI_OK when none runs).
 // XCD chunk of the longest-first order: one head's query tiles (nqt), so that
 // each XCD sorts and runs one head at a time and its L2 holds that head's
 // K/V blocks (HY long rollout: 0.687 against 0.706 ms with two heads mixed per
@@ -1490,11 +1546,14 @@ int xcd_chunk(int64_t tiles, int32_t nqt) {
   return (nqt > 0 && tiles > 0 && tiles % (8 * (int64_t)nqt) == 0) ? nqt : 0;
 }
 
+// Workspace use of one call: with LI_BSA_BALANCE (D = 128 kernels) the tile
+// order, built by bsa_order_kernel and no split; otherwise the split's partials
+// (D = 128, BS = 128).  Returns the launch status of the order kernel (LI_OK
+// when none runs).
 int plan_units(BsaArgs& a, int64_t tiles, int32_t D, int32_t block_size, void* workspace, int64_t workspace_bytes,
                int32_t flags, hipStream_t s) {
   a.ntiles = (int32_t)tiles;
-  a.xtiles = (int32_t)(tiles / 8);
-  a.xsplit = 0;
+  a.xwhole = a.xsplit = a.xparts = 0;
   a.part = nullptr;
   a.order = nullptr;
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0 || D != 128) return LI_OK;
@@ -1510,11 +1569,13 @@ int plan_units(BsaArgs& a, int64_t tiles, int32_t D, int32_t block_size, void* w
     return st;
   }
   if (block_size != 128) return LI_OK;
-  const int64_t r = split_per_xcd(tiles, device_cus());
-  if (r > 0 && workspace_bytes >= 8 * r * kPartBytesPerTile) {
-    a.xsplit = (int32_t)r;
-    a.part = static_cast<float*>(workspace);
-  }
+  const SplitPlan plan = plan_split(tiles, a.n_cols, device_cus(), workspace_bytes);
+  a.xwhole = plan.whole;
+  a.xsplit = plan.split;
+  a.xparts = plan.parts;
+  a.mg_split = magic16(plan.split > 0 ? plan.split : 1);
+  a.mg_parts = magic16(plan.parts > 0 ? plan.parts : 1);
+  if (plan.parts > 0) a.part = static_cast<float*>(workspace);
   return LI_OK;
 }
 
@@ -1526,7 +1587,23 @@ using namespace li;
 extern "C" int64_t li_bsa_fwd_workspace_size(int32_t B, int32_t NH, int32_t Lq, int32_t D, int32_t block_size) {
   if (B <= 0 || NH <= 0 || Lq <= 0 || D != 128 || block_size <= 0) return 0;
   const int64_t tiles = (int64_t)((Lq + block_size - 1) / block_size) * B * NH;
-  const int64_t split = block_size == 128 ? 8 * split_per_xcd(tiles, device_cus()) * kPartBytesPerTile : 0;
+  const int64_t c = device_cus() / 8, n = tiles / 8;
+  // Two pieces of each tile of a last round that is at most half full.
+  const int64_t r = c > 0 && device_cus() % 8 == 0 && tiles % 8 == 0 && n > c && 2 * (n % c) <= c ? n % c : 0;
+  const int64_t split = block_size == 128 ? 8 * r * 2 * kPartBytes : 0;
+  const int64_t ord = order_bytes(tiles);
+  return split > ord ? split : ord;
+}
+
+extern "C" int64_t li_bsa_fwd_workspace_size_cols(int32_t B, int32_t NH, int32_t Lq, int32_t D, int32_t block_size,
+                                                  int32_t n_cols) {
+  if (B <= 0 || NH <= 0 || Lq <= 0 || D != 128 || block_size <= 0 || n_cols < 0) return 0;
+  const int64_t tiles = (int64_t)((Lq + block_size - 1) / block_size) * B * NH;
+  int64_t split = 0;
+  if (block_size == 128) {
+    const SplitPlan p = plan_split(tiles, n_cols, device_cus(), kMaxPartBytes);
+    split = (int64_t)8 * p.split * p.parts * kPartBytes;
+  }
   const int64_t ord = order_bytes(tiles);
   return split > ord ? split : ord;
 }
@@ -1571,8 +1648,8 @@ extern "C" int li_bsa_fwd(int dtype, int32_t B, int32_t NH, int32_t Lq, int32_t 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int st = plan_units(a, tiles, D, block_size, workspace, workspace_bytes, flags, s);
   if (st != LI_OK) return st;
-  if (dtype == LI_DTYPE_BF16) return dispatch_bsa<Bf16>(a, block_size, D, (int)tiles, s);
-  return dispatch_bsa<F16>(a, block_size, D, (int)tiles, s);
+  if (dtype == LI_DTYPE_BF16) return dispatch_bsa<Bf16>(a, block_size, D, s);
+  return dispatch_bsa<F16>(a, block_size, D, s);
 }
 
 namespace {
@@ -1744,8 +1821,8 @@ extern "C" int li_bsa_fwd_gather(int dtype, int32_t B, int32_t NH, int32_t D, co
   hipStream_t s = static_cast<hipStream_t>(stream);
   st = plan_units(a, tiles, D, 128, workspace, workspace_bytes, flags, s);
   if (st != LI_OK) return st;
-  if (dtype == LI_DTYPE_BF16) return launch_bsa_gather<Bf16>(a, (int)tiles, s);
-  return launch_bsa_gather<F16>(a, (int)tiles, s);
+  if (dtype == LI_DTYPE_BF16) return launch_bsa_gather<Bf16>(a, s);
+  return launch_bsa_gather<F16>(a, s);
 }
 
 // Scratch of li_bsa_fwd_gather_noalloc: the tail split's partials or the
@@ -1797,15 +1874,15 @@ extern "C" int li_bsa_fwd_gather_noalloc(int dtype, int32_t B, int32_t NH, int32
                         out_strides, lse, false, (flags & LI_BSA_SORTED) != 0);
   if (st != LI_OK || tiles == 0) return st;
   // The workspace li_bsa_fwd_gather would use for this call must fit the scratch.
-  const int64_t need = li_bsa_fwd_workspace_size(B, NH, a.nqt * 128, D, 128);
+  const int64_t need = li_bsa_fwd_workspace_size_cols(B, NH, a.nqt * 128, D, 128, n_cols);
   if (need > kScratchBytes) return LI_ERR_TOO_LARGE;
   void* ws = scratch_ptr();
   if (!ws) return LI_ERR_LAUNCH;
   hipStream_t s = static_cast<hipStream_t>(stream);
   st = plan_units(a, tiles, D, 128, ws, need, flags, s);
   if (st != LI_OK) return st;
-  if (dtype == LI_DTYPE_BF16) return launch_bsa_gather<Bf16>(a, (int)tiles, s);
-  return launch_bsa_gather<F16>(a, (int)tiles, s);
+  if (dtype == LI_DTYPE_BF16) return launch_bsa_gather<Bf16>(a, s);
+  return launch_bsa_gather<F16>(a, s);
 }
 
 extern "C" int64_t li_bsa_fwd_noalloc_scratch_bytes(void) { return kScratchBytes; }
@@ -1853,7 +1930,7 @@ extern "C" int li_bsa_fwd_fp8(int32_t B, int32_t NH, int32_t Lq, int32_t Lk, int
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int st = plan_units(a, tiles, D, block_size, workspace, workspace_bytes, flags, s);
   if (st != LI_OK) return st;
-  return launch_bsa_fp8<false>(a, (int)tiles, s);
+  return launch_bsa_fp8<false>(a, s);
 }
 
 extern "C" int li_bsa_fwd_fp8_gather(int32_t B, int32_t NH, int32_t D, const void* q8, const float* q_scale,
@@ -1878,7 +1955,7 @@ extern "C" int li_bsa_fwd_fp8_gather(int32_t B, int32_t NH, int32_t D, const voi
   hipStream_t s = static_cast<hipStream_t>(stream);
   st = plan_units(a, tiles, D, 128, workspace, workspace_bytes, flags, s);
   if (st != LI_OK) return st;
-  return launch_bsa_fp8<true>(a, (int)tiles, s);
+  return launch_bsa_fp8<true>(a, s);
 }
 
 extern "C" int li_attn_fwd_dense(int dtype, int32_t B, int32_t NH, int32_t D, int32_t Lq, int32_t Lk, const void* q,
@@ -1955,6 +2032,6 @@ extern "C" int li_attn_fwd_dense(int dtype, int32_t B, int32_t NH, int32_t D, in
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int st = plan_units(a, tiles, D, 128, workspace, workspace_bytes, 0, s);
   if (st != LI_OK) return st;
-  if (dtype == LI_DTYPE_BF16) return launch_bsa_gather<Bf16, true>(a, (int)tiles, s);
-  return launch_bsa_gather<F16, true>(a, (int)tiles, s);
+  if (dtype == LI_DTYPE_BF16) return launch_bsa_gather<Bf16, true>(a, s);
+  return launch_bsa_gather<F16, true>(a, s);
 }

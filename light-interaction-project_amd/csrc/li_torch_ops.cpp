@@ -74,10 +74,13 @@ std::array<int64_t, N> strides(const at::Tensor& t) {
 }
 
 // Workspace of the attention launches: a caching-allocator buffer of the size
-// the library asks for on this device (tail split partials or tile order).
-at::Tensor workspace(const at::Tensor& like, int64_t B, int64_t NH, int64_t Lq, int64_t D, int64_t bs, bool want) {
+// the library asks for on this device (split partials or tile order) with
+// lists of n_cols columns.
+at::Tensor workspace(const at::Tensor& like, int64_t B, int64_t NH, int64_t Lq, int64_t D, int64_t bs, int64_t n_cols,
+                     bool want) {
   if (!want) return at::Tensor();
-  const int64_t bytes = li_bsa_fwd_workspace_size((int32_t)B, (int32_t)NH, (int32_t)Lq, (int32_t)D, (int32_t)bs);
+  const int64_t bytes = li_bsa_fwd_workspace_size_cols((int32_t)B, (int32_t)NH, (int32_t)Lq, (int32_t)D, (int32_t)bs,
+                                                       (int32_t)n_cols);
   if (bytes <= 0) return at::Tensor();
   return at::empty({(bytes + 3) / 4}, like.options().dtype(at::kFloat));
 }
@@ -360,7 +363,7 @@ at::Tensor bsa_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v
   on_device(q, out, "out");
   lists(indices, counts, B, NH, (Lq + block_size - 1) / block_size, q);
   at::Tensor lse = lse_or_empty(q, return_lse, B, NH, Lq);
-  at::Tensor ws = workspace(q, B, NH, Lq, D, block_size, split || balance);
+  at::Tensor ws = workspace(q, B, NH, Lq, D, block_size, indices.size(3), split || balance);
   const auto is = strides<4>(indices);
   const auto cs = strides<3>(counts);
   const int st = li_bsa_fwd(dtype_code(q), (int32_t)B, (int32_t)NH, (int32_t)Lq, (int32_t)Lk, (int32_t)D,
@@ -396,7 +399,7 @@ at::Tensor bsa_fwd_gather(const at::Tensor& q, const at::Tensor& k, const at::Te
   text(v_txt, num_txt_blk * bs, B, NH, D, "v_txt", q);
   lists(indices, counts, B, NH, nq, q);
   at::Tensor lse = lse_or_empty(q, return_lse, B, NH, nq * bs);
-  at::Tensor ws = workspace(q, B, NH, nq * bs, D, bs, split || balance);
+  at::Tensor ws = workspace(q, B, NH, nq * bs, D, bs, indices.size(3), split || balance);
   const at::Tensor kt = num_txt_blk > 0 && k_txt.has_value() ? *k_txt : at::Tensor();
   const at::Tensor vt = num_txt_blk > 0 && v_txt.has_value() ? *v_txt : at::Tensor();
   const auto qs = strides<4>(q);
@@ -433,7 +436,7 @@ at::Tensor attn_dense(const at::Tensor& q, const at::Tensor& k, const at::Tensor
   text(k_txt, (txt_len + 127) / 128 * 128, B, NH, D, "k_txt", q);
   text(v_txt, (txt_len + 127) / 128 * 128, B, NH, D, "v_txt", q);
   at::Tensor lse = lse_or_empty(q, return_lse, B, NH, nq * 128);
-  at::Tensor ws = workspace(q, B, NH, nq * 128, D, 128, split);
+  at::Tensor ws = workspace(q, B, NH, nq * 128, D, 128, (txt_len + 127) / 128 + (Lk + 127) / 128, split);
   const at::Tensor kt = txt_len > 0 && k_txt.has_value() ? *k_txt : at::Tensor();
   const at::Tensor vt = txt_len > 0 && v_txt.has_value() ? *v_txt : at::Tensor();
   const auto qs = strides<4>(q);
@@ -545,7 +548,7 @@ at::Tensor bsa_fwd_fp8(const at::Tensor& q8, const at::Tensor& q_scale, const at
   on_device(q8, out, "out");
   lists(indices, counts, B, NH, (Lq + block_size - 1) / block_size, q8);
   at::Tensor lse = lse_or_empty(v, return_lse, B, NH, Lq);
-  at::Tensor ws = workspace(v, B, NH, Lq, D, block_size, split || balance);
+  at::Tensor ws = workspace(v, B, NH, Lq, D, block_size, indices.size(3), split || balance);
   const auto is = strides<4>(indices);
   const auto cs = strides<3>(counts);
   const int st = li_bsa_fwd_fp8((int32_t)B, (int32_t)NH, (int32_t)Lq, (int32_t)Lk, (int32_t)D, q8.data_ptr(),
@@ -590,7 +593,7 @@ at::Tensor bsa_fwd_fp8_gather(const at::Tensor& q8, const at::Tensor& q_scale, c
   text(v_txt, num_txt_blk * 128, B, NH, D, "v_txt", v);
   lists(indices, counts, B, NH, nq, v);
   at::Tensor lse = lse_or_empty(v, return_lse, B, NH, nq * 128);
-  at::Tensor ws = workspace(v, B, NH, nq * 128, D, 128, true);
+  at::Tensor ws = workspace(v, B, NH, nq * 128, D, 128, indices.size(3), true);
   const at::Tensor vt = num_txt_blk > 0 && v_txt.has_value() ? *v_txt : at::Tensor();
   const auto vs = strides<4>(v);
   const auto os = strides<4>(out);

@@ -16,7 +16,7 @@ import os
 import torch  # noqa: F401  (must precede the CDLL below)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libli_sparse_attn.so")
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 LI_OK = 0
 LI_ERR_INVALID_ARG = -1
@@ -76,6 +76,7 @@ SIGNATURES = {
     "li_bsa_fwd": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64p, _i32,
                                   _vp, _i64p, ctypes.c_float, _i32, _vp, _vp, _vp, _i64, _i32, _vp]),
     "li_bsa_fwd_workspace_size": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32]),
+    "li_bsa_fwd_workspace_size_cols": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "li_bsa_fwd_gather": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _vp,
                                          _i32, ctypes.POINTER(TileGeom), ctypes.POINTER(TileGeom), _vp, _i64p, _i32,
                                          _vp, _i64p, ctypes.c_float, _vp, _i64p, _vp, _vp, _i64, _i32, _vp]),
