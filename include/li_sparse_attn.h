@@ -102,9 +102,9 @@ int li_pool(int dtype, int32_t B, int32_t NH, int32_t D,
  * job 0 (src0, mean0, pool_off0, geom0) and job 1 (src1, ...) as li_pool each,
  * same bits.  Replaces the two pool calls the reference makes per call, the
  * launch_q_prep and launch_kv_prep means (HYAR:58-70, 110-122, called at
- * HYAR:330-361), for the fused path.  When one job has no blocks or their
- * sources differ in vector access (16-byte aligned unit-stride rows), the
- * jobs are launched one after the other.
+ * HYAR:330-361), for the fused path.  When the sources differ in vector
+ * access (16-byte aligned unit-stride rows), the jobs are launched one after
+ * the other.
  *   mean1_normalized: optional (NULL), same shape and strides as mean1: each
  *     pooled row of job 1 divided by its L2 norm as the cosine metric of
  *     li_block_mask normalises a key pool row (HYAR:250-252), same bits; the
@@ -119,6 +119,32 @@ int li_pool_pair(int dtype, int32_t B, int32_t NH, int32_t D,
                  const void* src1, const int64_t src1_strides[4],
                  void* mean1, const int64_t mean1_strides[4], int64_t pool_off1,
                  const li_tile_geom* geom1, void* mean1_normalized, void* stream);
+
+/*
+ * Everything that an attention call prepares of its tensors in a single launch
+ * (two when only some of the jobs can be moved with vector accesses): up to 5
+ * jobs, each the gather of one (B, NH, L, D) tensor into tiles, its mean pool,
+ * or both, as li_q_prep / li_pool / li_tile_prep_fp8 do them, bit for bit.
+ * Replaces the launch_q_prep, launch_kv_prep and text F.pad / copy calls of one
+ * run_sparse_attention call (HYAR:330-348).  A text of n tokens is padded into
+ * blocks of BS rows by the geometry T = 1, H = 1, W = n, tile (1, 1, BS), nh =
+ * 1, nw = ceil(n / BS).
+ */
+typedef struct li_prep_job {
+  const void* src;
+  int64_t src_strides[4];
+  li_tile_geom geom;
+  void* dst;                /* tiles (B, NH, nblk, BS, D) at block (blk + dst_off), or NULL */
+  int64_t dst_strides[5];
+  int64_t dst_off;
+  float* scales;            /* non-NULL: dst takes e4m3 codes, scales (B, NH, nblk) at (blk + dst_off) */
+  int64_t scale_strides[3];
+  void* mean;               /* pool (B, NH, nblk, D) at block (blk + pool_off), or NULL */
+  void* mean_normalized;    /* as li_pool_pair's, strides of mean, or NULL */
+  int64_t mean_strides[4];
+  int64_t pool_off;
+} li_prep_job;
+int li_prep(int dtype, int32_t B, int32_t NH, int32_t D, const li_prep_job* jobs, int32_t n_jobs, void* stream);
 
 /*
  * Untile scatter.  Replaces launch_untile(src, dst, T, H, W, tt, th, tw, nh, nw)

@@ -21,6 +21,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <array>
 #include <cmath>
 #include <string>
@@ -215,6 +216,120 @@ void pool_pair(const at::Tensor& src0, at::Tensor& mean0, int64_t off0, c10::Int
         li_pool_pair(dtype_code(src0), (int32_t)src0.size(0), (int32_t)src0.size(1), (int32_t)src0.size(3),
                      src0.data_ptr(), s0.data(), mean0.data_ptr(), m0.data(), off0, &g0, src1.data_ptr(), s1.data(),
                      mean1.data_ptr(), m1.data(), off1, &g1, mean1_n, stream_of(src0)));
+}
+
+typedef c10::optional<at::Tensor> OptTensor;
+
+bool given(const OptTensor& t) { return t.has_value() && t->defined(); }
+
+// One li_prep job: `src` over geometry `g`, tiles (16-bit, or e4m3 codes with
+// `scale`) at block dst_off of `tiles`, pool at block pool_off of `mean`.
+li_prep_job prep_job(const at::Tensor& src, const li_tile_geom& g, const at::Tensor* tiles, const at::Tensor* scale,
+                     int64_t dst_off, const at::Tensor* mean, const at::Tensor* mean_n, int64_t pool_off,
+                     const char* name, const at::Tensor& like) {
+  const int64_t B = like.size(0), NH = like.size(1), D = like.size(3);
+  TORCH_CHECK(dst_off >= 0 && pool_off >= 0, name, ": block offsets must be >= 0");
+  rows4(src, B, NH, tokens_of(g), D, name, &like);
+  li_prep_job j{};
+  j.src = src.data_ptr();
+  std::copy_n(src.strides().data(), 4, j.src_strides);
+  j.geom = g;
+  if (tiles) {
+    tiles5(*tiles, B, NH, blocks_of(g) + dst_off, block_size_of(g), D, "tiles", like);
+    if (scale) {
+      codes(*tiles, "tiles");
+      scales3(*scale, B, NH, blocks_of(g) + dst_off, "scales", like);
+      j.scales = scale->data_ptr<float>();
+      std::copy_n(scale->strides().data(), 3, j.scale_strides);
+    } else {
+      TORCH_CHECK(tiles->scalar_type() == like.scalar_type(), "tiles must be ", like.scalar_type());
+    }
+    j.dst = tiles->data_ptr();
+    std::copy_n(tiles->strides().data(), 5, j.dst_strides);
+    j.dst_off = dst_off;
+  }
+  if (mean) {
+    rows4(*mean, B, NH, blocks_of(g) + pool_off, D, "pool", &like);
+    j.mean = mean->data_ptr();
+    std::copy_n(mean->strides().data(), 4, j.mean_strides);
+    j.pool_off = pool_off;
+    if (mean_n) {
+      TORCH_CHECK(mean_n->sizes() == mean->sizes() && mean_n->strides() == mean->strides() &&
+                      mean_n->scalar_type() == mean->scalar_type() && mean_n->device() == mean->device(),
+                  "the normalised pool must match the pool in shape, strides, dtype and device");
+      j.mean_normalized = mean_n->data_ptr();
+    }
+  }
+  return j;
+}
+
+// A text of `n` tokens as blocks of bs rows, padded with zeros.
+li_tile_geom text_geom(int64_t n, int64_t bs) {
+  return li_tile_geom{1, 1, (int32_t)n, 1, 1, (int32_t)bs, 1, (int32_t)((n + bs - 1) / bs)};
+}
+
+// Padded text rows (B, NH, blocks * bs, D), contiguous, as (B, NH, blocks, bs, D) tiles.
+at::Tensor text_tiles(const at::Tensor& t, int64_t blocks, int64_t bs, const char* name) {
+  TORCH_CHECK(t.is_contiguous() && t.dim() == 4 && t.size(2) == blocks * bs, name, " must be contiguous, ", blocks * bs,
+              " rows, got ", t.sizes());
+  return t.view({t.size(0), t.size(1), blocks, bs, t.size(3)});
+}
+
+const at::Tensor* opt(const OptTensor& t) { return given(t) ? &*t : nullptr; }
+
+// The preparation of one attention call in one launch: the query pool (and
+// tiles), the key pool (and tiles), the value tiles, and the text in the
+// leading blocks of k_tiles / v_tiles where these are given, else padded into
+// txt_k / txt_v.  k and v start at block `first` of the key grid.
+void prep(const at::Tensor& q, const OptTensor& q_tiles, const OptTensor& q_scale, at::Tensor& q_pool,
+          c10::IntArrayRef q_geom, const at::Tensor& k, const at::Tensor& v, const OptTensor& k_tiles,
+          const OptTensor& k_scale, const OptTensor& v_tiles, at::Tensor& k_pool, const OptTensor& k_pool_n,
+          int64_t first, c10::IntArrayRef k_geom, int64_t num_txt_blk, const OptTensor& k_txt, const OptTensor& v_txt,
+          const OptTensor& txt_k, const OptTensor& txt_v) {
+  gpu(q, "q");
+  rank(q, 4, "q");
+  c10::DeviceGuard guard(q.device());
+  const li_tile_geom gq = geom_of(q_geom), gk = geom_of(k_geom);
+  const int64_t bs = block_size_of(gq);
+  TORCH_CHECK(block_size_of(gk) == bs, "q and k tiles differ in size");
+  TORCH_CHECK(first >= 0 && num_txt_blk >= 0, "block offsets must be >= 0");
+  li_prep_job jobs[5];
+  int n = 0;
+  if (given(k_txt) && k_txt->size(2) > 0) {
+    TORCH_CHECK(given(v_txt) && v_txt->sizes() == k_txt->sizes(), "v_txt must have k_txt's shape");
+    const li_tile_geom g = text_geom(k_txt->size(2), bs);
+    TORCH_CHECK(g.nw == num_txt_blk, "num_txt_blk must be ", g.nw);
+    at::Tensor kt, vt;
+    if (given(k_tiles)) kt = *k_tiles;
+    else if (given(txt_k)) kt = text_tiles(*txt_k, num_txt_blk, bs, "txt_k");
+    if (given(v_tiles)) vt = *v_tiles;
+    else if (given(txt_v)) vt = text_tiles(*txt_v, num_txt_blk, bs, "txt_v");
+    if (kt.defined())
+      jobs[n++] = prep_job(*k_txt, g, &kt, given(k_tiles) ? opt(k_scale) : nullptr, 0, nullptr, nullptr, 0, "k_txt", q);
+    if (vt.defined()) jobs[n++] = prep_job(*v_txt, g, &vt, nullptr, 0, nullptr, nullptr, 0, "v_txt", q);
+  }
+  jobs[n++] = prep_job(q, gq, opt(q_tiles), opt(q_scale), 0, &q_pool, nullptr, 0, "q", q);
+  if (blocks_of(gk) > 0)  // none when every key block is kept from an earlier call
+    jobs[n++] = prep_job(k, gk, opt(k_tiles), opt(k_scale), num_txt_blk + first, &k_pool, opt(k_pool_n), first, "k", q);
+  if (given(v_tiles) && blocks_of(gk) > 0)
+    jobs[n++] = prep_job(v, gk, opt(v_tiles), nullptr, num_txt_blk + first, nullptr, nullptr, 0, "v", q);
+  check("li_prep", li_prep(dtype_code(q), (int32_t)q.size(0), (int32_t)q.size(1), (int32_t)q.size(3), jobs, n,
+                           stream_of(q)));
+}
+
+// Text keys and values padded with zeros into whole blocks, in one launch.
+void pad_text(const at::Tensor& k_txt, const at::Tensor& v_txt, at::Tensor& k_out, at::Tensor& v_out, int64_t bs) {
+  gpu(k_txt, "k_txt");
+  rank(k_txt, 4, "k_txt");
+  c10::DeviceGuard guard(k_txt.device());
+  TORCH_CHECK(v_txt.sizes() == k_txt.sizes(), "v_txt must have k_txt's shape");
+  TORCH_CHECK(bs > 0 && k_txt.size(2) > 0, "block size and text length must be positive");
+  const li_tile_geom g = text_geom(k_txt.size(2), bs);
+  const at::Tensor kt = text_tiles(k_out, g.nw, bs, "k_out"), vt = text_tiles(v_out, g.nw, bs, "v_out");
+  const li_prep_job jobs[2] = {prep_job(k_txt, g, &kt, nullptr, 0, nullptr, nullptr, 0, "k_txt", k_txt),
+                               prep_job(v_txt, g, &vt, nullptr, 0, nullptr, nullptr, 0, "v_txt", k_txt)};
+  check("li_prep", li_prep(dtype_code(k_txt), (int32_t)k_txt.size(0), (int32_t)k_txt.size(1), (int32_t)k_txt.size(3),
+                           jobs, 2, stream_of(k_txt)));
 }
 
 void q_prep(const at::Tensor& src, at::Tensor& dst, at::Tensor& mean, c10::IntArrayRef geom) {
@@ -616,6 +731,11 @@ TORCH_LIBRARY(li, m) {
   m.def("pool(Tensor src, Tensor(a!) mean, int pool_off, int[] geom) -> ()");
   m.def("pool_pair(Tensor src0, Tensor(a!) mean0, int pool_off0, int[] geom0, Tensor src1, Tensor(b!) mean1, "
         "int pool_off1, int[] geom1, Tensor(c!)? mean1_normalized=None) -> ()");
+  m.def("prep(Tensor q, Tensor(a!)? q_tiles, Tensor(b!)? q_scale, Tensor(c!) q_pool, int[] q_geom, Tensor k, Tensor v, "
+        "Tensor(d!)? k_tiles, Tensor(e!)? k_scale, Tensor(f!)? v_tiles, Tensor(g!) k_pool, Tensor(h!)? k_pool_n, "
+        "int first, int[] k_geom, int num_txt_blk, Tensor? k_txt, Tensor? v_txt, Tensor(i!)? txt_k, "
+        "Tensor(j!)? txt_v) -> ()");
+  m.def("pad_text(Tensor k_txt, Tensor v_txt, Tensor(a!) k_out, Tensor(b!) v_out, int bs) -> ()");
   m.def("q_prep(Tensor src, Tensor(a!) dst, Tensor(b!) mean, int[] geom) -> ()");
   m.def("kv_prep(Tensor k_src, Tensor v_src, Tensor(a!) k_dst, Tensor(b!) v_dst, Tensor(c!) k_mean, int dst_off, "
         "int pool_off, int[] geom) -> ()");
@@ -644,6 +764,8 @@ TORCH_LIBRARY(li, m) {
 TORCH_LIBRARY_IMPL(li, CUDA, m) {
   m.impl("pool", &pool);
   m.impl("pool_pair", &pool_pair);
+  m.impl("prep", &prep);
+  m.impl("pad_text", &pad_text);
   m.impl("q_prep", &q_prep);
   m.impl("kv_prep", &kv_prep);
   m.impl("untile", &untile);

@@ -199,6 +199,36 @@ def pool_pair(src0, mean0, pool_off0, geom0, src1, mean1, pool_off1, geom1, mean
     _run(ops.pool_pair, src0, mean0, int(pool_off0), gs[0], src1, mean1, int(pool_off1), gs[1], mean1_normalized)
 
 
+def prep(q, q_pool, geom_q, k, v, k_pool, first, geom_k, *, q_tiles=None, q_scale=None, k_tiles=None, k_scale=None,
+         v_tiles=None, k_pool_n=None, num_txt_blk=0, text=None, padded_text=(None, None)):
+    """The preparation of one attention call in one launch (see li_prep).
+
+    Pools of ``q`` and ``k`` (geom = (T, H, W, tt, th, tw, nh, nw) of each); tiles of them and of ``v`` where tile
+    buffers are given, as e4m3 codes where a scale buffer is.  ``k`` and ``v`` start at block ``first`` of the key
+    grid.  ``text`` = (k_txt, v_txt), any length and strides, zero-padded into the ``num_txt_blk`` leading blocks of
+    ``k_tiles`` / ``v_tiles`` where these are given, else into ``padded_text`` (contiguous rows, or None to leave it).
+    """
+    _device_check(q, k, v, q_pool, k_pool)
+    _same_dtype(q, k, v, q_pool, k_pool)
+    dtype_code(q)
+    if v_tiles is not None and tuple(v.shape) != tuple(k.shape):
+        raise ValueError(f"K/V source shapes differ: {tuple(k.shape)} vs {tuple(v.shape)}")
+    k_txt, v_txt = text if text is not None else (None, None)
+    _run(ops.prep, q, q_tiles, q_scale, q_pool, geom_q, k, v, k_tiles, k_scale, v_tiles, k_pool, k_pool_n, first, geom_k,
+         num_txt_blk, k_txt, v_txt, *padded_text)
+
+
+def pad_text(k_txt, v_txt, bs):
+    """(k_txt, v_txt) as contiguous rows zero-padded to whole blocks of ``bs``, in one launch (themselves if they are)."""
+    n = k_txt.shape[2]
+    if n % bs == 0 and k_txt.is_contiguous() and v_txt.is_contiguous():
+        return k_txt, v_txt
+    shape = (*k_txt.shape[:2], ceil_div(n, bs) * bs, k_txt.shape[3])
+    kt, vt = k_txt.new_empty(shape), v_txt.new_empty(shape)
+    _run(ops.pad_text, k_txt, v_txt, kt, vt, bs)
+    return kt, vt
+
+
 def fused_supported(D, tile, latent_hw):
     """Whether li_bsa_fwd_gather covers this shape.
 
@@ -543,9 +573,7 @@ def attn_dense(q, k, v, k_txt=None, v_txt=None, sm_scale=None, return_lse=False,
         _same_dtype(q, k_txt, v_txt)
         if tuple(k_txt.shape) != (B, NH, txt_len, D) or tuple(v_txt.shape) != (B, NH, txt_len, D):
             raise ValueError(f"text K/V shapes {tuple(k_txt.shape)} / {tuple(v_txt.shape)} do not match q")
-        pad = (-txt_len) % 128
-        kt = (torch.nn.functional.pad(k_txt, (0, 0, 0, pad)) if pad else k_txt).contiguous()
-        vt = (torch.nn.functional.pad(v_txt, (0, 0, 0, pad)) if pad else v_txt).contiguous()
+        kt, vt = pad_text(k_txt, v_txt, 128)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D)
     if out is None:

@@ -52,6 +52,12 @@ class TileGeom(ctypes.Structure):
                 ("nh", _i32), ("nw", _i32)]
 
 
+class PrepJob(ctypes.Structure):
+    _fields_ = [("src", _vp), ("src_strides", _i64 * 4), ("geom", TileGeom), ("dst", _vp), ("dst_strides", _i64 * 5),
+                ("dst_off", _i64), ("scales", _vp), ("scale_strides", _i64 * 3), ("mean", _vp),
+                ("mean_normalized", _vp), ("mean_strides", _i64 * 4), ("pool_off", _i64)]
+
+
 class MaskParams(ctypes.Structure):
     _fields_ = [("metric", _i32), ("budget_mode", _i32), ("topk_ratio", ctypes.c_double),
                 ("min_budget", _i32), ("n_recent", _i32), ("force_diag", _i32), ("force_sink", _i32),
@@ -98,6 +104,7 @@ SIGNATURES = {
                                          _i64p, _vp, _vp, _i32, ctypes.c_float, _vp, _i64p, _vp, _vp, _i64, _vp]),
     "li_pool": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _vp, _i64p, _vp, _i64p, _i64,
                                ctypes.POINTER(TileGeom), _vp]),
+    "li_prep": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, ctypes.POINTER(PrepJob), _i32, _vp]),
     "li_pool_pair": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _vp, _i64p, _vp, _i64p, _i64,
                                     ctypes.POINTER(TileGeom), _vp, _i64p, _vp, _i64p, _i64,
                                     ctypes.POINTER(TileGeom), _vp, _vp]),

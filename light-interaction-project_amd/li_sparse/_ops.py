@@ -11,6 +11,7 @@ operators trace under FakeTensor / meta tensors (torch.compile,
 torch.export).  Loading fails loudly when either library is missing.
 
 Operators (schemas in csrc/li_torch_ops.cpp): ``pool``, ``pool_pair``,
+``prep`` (everything a call prepares of its tensors, in one launch), ``pad_text``,
 ``q_prep``, ``kv_prep``, ``untile`` (tile gather / pool / scatter,
 ar_sparse_operation.py:166-218), ``block_mask`` (fast_generate_indices /
 generate_prefill_indices, ar_sparse_operation.py:223-284,
@@ -73,6 +74,17 @@ def _pool_fake(src, mean, pool_off, geom):
 
 @torch.library.register_fake("li::pool_pair")
 def _pool_pair_fake(src0, mean0, pool_off0, geom0, src1, mean1, pool_off1, geom1, mean1_normalized=None):
+    return None
+
+
+@torch.library.register_fake("li::prep")
+def _prep_fake(q, q_tiles, q_scale, q_pool, q_geom, k, v, k_tiles, k_scale, v_tiles, k_pool, k_pool_n, first, k_geom,
+               num_txt_blk, k_txt, v_txt, txt_k, txt_v):
+    return None
+
+
+@torch.library.register_fake("li::pad_text")
+def _pad_text_fake(k_txt, v_txt, k_out, v_out, bs):
     return None
 
 

@@ -126,113 +126,80 @@ def context_of(sparse_params, block_idx):
     return cache, block_idx, int(sparse_params.get("context_frames", 0))
 
 
-def _pad_text(x, g, text_len):
-    pad = g.num_txt_blk * g.bs - text_len
-    return (F.pad(x, (0, 0, 0, pad)) if pad > 0 else x).contiguous()
+def _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm):
+    """What one call prepares of its tensors, in one launch (li_prep): a dict of the buffers.
 
-
-def _k_side(path, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, B, NH, D, dev, dt, q_pool_job=None, k_norm=False):
-    """Key-side buffers of one call: text blocks, then the visual blocks from the first uncached frame.
-
-    path: "fused" (K pool; padded text K/V), "fused_fp8" (e4m3 K tiles + scales, K pool; padded text V),
-    "tiled" (K/V tiles, K pool), "tiled_fp8" (e4m3 K tiles + scales, V tiles, K pool).
-    q_pool_job: (q, q_pool, pool_off, geometry) of the query pool, taken in the same launch as the K pool on
-    the fused path (li_pool_pair), or on its own when there is no K pool to take (every frame cached).
-    k_norm: on the fused path, also keep the K pool's rows normalised for the cosine selection (written by
-    the same launch, ``k_pool_n``; the selection takes it as ``k_pool_normalized``).
+    path: "fused" (pools; padded text K/V), "fused_fp8" (e4m3 Q and K tiles + scales, pools; padded text V), "tiled"
+    (Q, K, V tiles, pools), "tiled_fp8" (e4m3 Q and K tiles + scales, V tiles, pools).  Query-side buffers are the
+    call's own; key-side ones (text blocks, then the visual blocks from the first uncached frame) are the
+    ContextCache's where there is one.  k_norm: also keep the K pool's rows normalised for the cosine selection
+    (``k_pool_n``; the selection takes it as ``k_pool_normalized``).
     """
+    B, NH, _, D = q.shape
+    dt = q.dtype
+    fp8, tiled = path in ("fused_fp8", "tiled_fp8"), path in ("tiled", "tiled_fp8")
+    if path == "fused" and text_len > 0:
+        _core._same_dtype(q, k_txt, v_txt)
+    elif text_len > 0:
+        k_txt, v_txt = k_txt.to(dt), v_txt.to(dt)
     cache, layer, cframes = ctx if ctx is not None else (None, None, 0)
     cf = min((max(cframes, 0) // g.tt) * g.tt, g.T_k) if cache is not None else 0
-    k_norm = bool(k_norm) and path == "fused"
-    key = (path, layer, B, NH, D, dt, str(dev), g, text_len, cf, k_norm)
+    key = (path, layer, B, NH, D, dt, str(q.device), g, text_len, cf, bool(k_norm)) if cache is not None else None
     bufs = cache._entries.get(key) if cache is not None else None
     first = cf if bufs is not None else 0
-    nkb = g.num_txt_blk + g.nk_blk
+    text, padded = None, (None, None)
     if bufs is None:
-        bufs = {"k_pool": torch.empty((B, NH, g.nk_blk, D), device=dev, dtype=dt), "k_pool_n": None}
+        nkb = g.num_txt_blk + g.nk_blk
+        bufs = dict.fromkeys(("k_pool_n", "k8", "k_scale", "k_all", "v_all", "kt", "vt"))
+        bufs["k_pool"] = q.new_empty((B, NH, g.nk_blk, D))
         if k_norm:
             bufs["k_pool_n"] = torch.empty_like(bufs["k_pool"])
-        if path in ("fused_fp8", "tiled_fp8"):
-            bufs["k8"] = torch.empty((B, NH, nkb, g.bs, D), device=dev, dtype=_core.FP8)
-            bufs["k_scale"] = torch.empty((B, NH, nkb), device=dev, dtype=torch.float32)
+        if fp8:
+            bufs["k8"] = q.new_empty((B, NH, nkb, g.bs, D), dtype=_core.FP8)
+            bufs["k_scale"] = q.new_empty((B, NH, nkb), dtype=torch.float32)
         if path == "tiled":
-            bufs["k_all"] = torch.empty((B, NH, nkb, g.bs, D), device=dev, dtype=dt)
-        if path in ("tiled", "tiled_fp8"):
-            bufs["v_all"] = torch.empty((B, NH, nkb, g.bs, D), device=dev, dtype=dt)
-        bufs["kt"] = bufs["vt"] = None
+            bufs["k_all"] = q.new_empty((B, NH, nkb, g.bs, D))
+        if tiled:
+            bufs["v_all"] = q.new_empty((B, NH, nkb, g.bs, D))
         if text_len > 0:
-            kt, vt = _pad_text(k_txt, g, text_len), _pad_text(v_txt, g, text_len)
+            text = (k_txt, v_txt)
+            # Whole blocks of text are read where they are.
+            whole = text_len % g.bs == 0
             if path == "fused":
-                bufs["kt"], bufs["vt"] = kt, vt
-            elif path == "fused_fp8":
-                bufs["vt"] = vt
-            if path in ("fused_fp8", "tiled_fp8"):
-                # Contiguous text blocks: the trivial grid T = blocks, H = 1, W = BS, tile (1, 1, BS).
-                _core.tile_prep_fp8(kt, bufs["k8"], bufs["k_scale"], None, 0, 0, g.num_txt_blk, 1, g.bs, 1, 1, g.bs,
-                                    1, 1)
-            if path == "tiled":
-                bufs["k_all"][:, :, :g.num_txt_blk].copy_(kt.view(B, NH, g.num_txt_blk, g.bs, D))
-            if path in ("tiled", "tiled_fp8"):
-                bufs["v_all"][:, :, :g.num_txt_blk].copy_(vt.view(B, NH, g.num_txt_blk, g.bs, D))
-        if cache is not None:
-            cache._entries[key] = bufs
-    T = g.T_k - first
-    if T > 0:
-        fb = (first // g.tt) * g.nh * g.nw
-        tok = first * g.H * g.W
-        kv, vv = k_vis[:, :, tok:], v_vis[:, :, tok:]
-        geo = (T, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw)
-        if path == "fused" and q_pool_job is not None:
-            _core.pool_pair(*q_pool_job, kv, bufs["k_pool"], fb, geo, mean1_normalized=bufs["k_pool_n"])
-            q_pool_job = None
-        elif path == "fused":
-            if k_norm:
-                raise ValueError("the normalised key pool is written with the query pool (li_pool_pair)")
-            _core.pool(kv, bufs["k_pool"], fb, *geo)
-        elif path == "fused_fp8":
-            _core.tile_prep_fp8(kv, bufs["k8"], bufs["k_scale"], bufs["k_pool"], g.num_txt_blk + fb, fb, *geo)
-        elif path == "tiled":
-            _core.kv_prep(kv, vv, bufs["k_all"], bufs["v_all"], bufs["k_pool"], g.num_txt_blk + fb, fb, *geo)
-        else:
-            _core.kv_prep_fp8(kv, vv, bufs["k8"], bufs["k_scale"], bufs["v_all"], bufs["k_pool"], g.num_txt_blk + fb,
-                              fb, *geo)
-    if q_pool_job is not None:
-        src, mean, off, qgeo = q_pool_job
-        _core.pool(src, mean, off, *qgeo)
-    return bufs
+                bufs["kt"], keep_k = _text_rows(k_txt, g, whole)
+                padded = (None if keep_k else bufs["kt"], None)
+            if not tiled:
+                bufs["vt"], keep_v = _text_rows(v_txt, g, whole)
+                padded = (padded[0], None if keep_v else bufs["vt"])
+    out = dict(bufs, q_pool=q.new_empty((B, NH, g.nq_blk, D)), q_tiles=None, q_scale=None)
+    if fp8:
+        out["q_tiles"] = q.new_empty((B, NH, g.nq_blk, g.bs, D), dtype=_core.FP8)
+        out["q_scale"] = q.new_empty((B, NH, g.nq_blk), dtype=torch.float32)
+    elif tiled:
+        out["q_tiles"] = q.new_empty((B, NH, g.nq_blk, g.bs, D))
+    if first > 0:
+        k_vis, v_vis = k_vis[:, :, first * g.H * g.W:], v_vis[:, :, first * g.H * g.W:]
+    rest = (g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw)
+    _core.prep(q, out["q_pool"], (g.T_q, *rest), k_vis, v_vis, bufs["k_pool"], (first // g.tt) * g.nh * g.nw,
+               (g.T_k - first, *rest), q_tiles=out["q_tiles"], q_scale=out["q_scale"],
+               k_tiles=bufs["k8"] if fp8 else bufs["k_all"], k_scale=bufs["k_scale"], v_tiles=bufs["v_all"],
+               k_pool_n=bufs["k_pool_n"], num_txt_blk=g.num_txt_blk, text=text, padded_text=padded)
+    if cache is not None:
+        cache._entries[key] = bufs
+    return out
 
 
-def _select(select, q_pool, kb, text_len, g):
+def _text_rows(x, g, whole):
+    """(padded text buffer, True if it is ``x`` itself)."""
+    if whole and x.is_contiguous():
+        return x, True
+    return x.new_empty((*x.shape[:2], g.num_txt_blk * g.bs, x.shape[3])), False
+
+
+def _select(select, kb, text_len, g):
     """``select`` on the call's pools; the normalised key pool goes along only when the call wrote one."""
-    kw = {} if kb.get("k_pool_n") is None else {"k_pool_normalized": kb["k_pool_n"]}
-    return select(q_pool, kb["k_pool"], text_len, (g.nt_q, g.nh, g.nw), (g.nt_k, g.nh, g.nw), **kw)
-
-
-def _fused(q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, out_dtype, events, balance, ctx, sorted_lists,
-           k_norm=False):
-    """Pools, block selection, then one kernel that gathers, attends and untiles."""
-    B, NH, _, D = q.shape
-    dev, dt = q.device, q.dtype
-    _stage(events, "alloc_start")
-    q_pool = torch.empty((B, NH, g.nq_blk, D), device=dev, dtype=dt)
-    o_out = torch.empty_like(q)
-    _stage(events, "alloc_end")
-    _stage(events, "prep_start")
-    q_job = (q, q_pool, 0, (g.T_q, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw))
-    kb = _k_side("fused", k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, B, NH, D, dev, dt, q_pool_job=q_job,
-                 k_norm=k_norm)
-    _stage(events, "prep_end")
-    _stage(events, "index_start")
-    indices, counts = _select(select, q_pool, kb, text_len, g)
-    _stage(events, "index_end")
-    _stage(events, "attn_start")
-    _core.bsa_forward_gather(q, k_vis, v_vis, kb["kt"], kb["vt"], g.num_txt_blk, g.T_q, g.T_k, g.H, g.W, g.tt, g.th,
-                             g.tw, g.nh, g.nw, indices, counts, 1.0 / math.sqrt(D), o_out, balance=balance,
-                             sorted_lists=sorted_lists)
-    _stage(events, "attn_end")
-    _stage(events, "untile_start")
-    _stage(events, "untile_end")
-    return o_out if o_out.dtype == out_dtype else o_out.to(out_dtype)
+    kw = {} if kb["k_pool_n"] is None else {"k_pool_normalized": kb["k_pool_n"]}
+    return select(kb["q_pool"], kb["k_pool"], text_len, (g.nt_q, g.nh, g.nw), (g.nt_k, g.nh, g.nw), **kw)
 
 
 def fp8_supported(D, tile):
@@ -240,64 +207,42 @@ def fp8_supported(D, tile):
     return D == 128 and tile[0] * tile[1] * tile[2] == 128
 
 
-def _q_fp8(q, g, B, NH, D, dev):
-    q8 = torch.empty((B, NH, g.nq_blk, g.bs, D), device=dev, dtype=_core.FP8)
-    q_scale = torch.empty((B, NH, g.nq_blk), device=dev, dtype=torch.float32)
-    q_pool = torch.empty((B, NH, g.nq_blk, D), device=dev, dtype=q.dtype)
-    _core.tile_prep_fp8(q, q8, q_scale, q_pool, 0, 0, g.T_q, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw)
-    return q8, q_scale, q_pool
-
-
-def _tiled_fp8(q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, out_dtype, events, balance, ctx, sorted_lists):
-    """Tiled sequence with Q and K quantized to e4m3 per tile block (scale amax / 448) in their gathers.
-
-    The pools (and so the block selection) are those of the bf16 path; V, P V and the output stay bf16.
-    """
+def _call(path, q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, events, balance, ctx, sorted_lists, k_norm):
+    """Preparation, block selection, attention, and the untile of the tiled paths."""
     B, NH, _, D = q.shape
-    dev = q.device
-    _stage(events, "alloc_start")
-    _stage(events, "alloc_end")
-    _stage(events, "prep_start")
-    q8, q_scale, q_pool = _q_fp8(q, g, B, NH, D, dev)
-    kb = _k_side("tiled_fp8", k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, B, NH, D, dev, q.dtype)
-    _stage(events, "prep_end")
-    _stage(events, "index_start")
-    indices, counts = _select(select, q_pool, kb, text_len, g)
-    _stage(events, "index_end")
-    _stage(events, "attn_start")
-    o_flat = _core.bsa_forward_fp8(q8.flatten(2, 3), q_scale, kb["k8"].flatten(2, 3), kb["k_scale"],
-                                   kb["v_all"].flatten(2, 3), indices, counts, 1.0 / math.sqrt(D), g.bs,
-                                   balance=balance)
-    _stage(events, "attn_end")
-    _stage(events, "untile_start")
-    o_out = torch.empty_like(q)
-    _core.untile(o_flat.view(B, NH, g.nq_blk, g.bs, D), o_out, g.T_q, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw)
-    _stage(events, "untile_end")
-    return o_out if o_out.dtype == out_dtype else o_out.to(out_dtype)
-
-
-def _fused_fp8(q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, out_dtype, events, balance, ctx, sorted_lists):
-    """e4m3 Q/K tiles from the quantizing gathers, then one kernel that reads V and writes O in token order."""
-    B, NH, _, D = q.shape
-    dev = q.device
+    scale = 1.0 / math.sqrt(D)
     _stage(events, "alloc_start")
     o_out = torch.empty_like(q)
     _stage(events, "alloc_end")
     _stage(events, "prep_start")
-    q8, q_scale, q_pool = _q_fp8(q, g, B, NH, D, dev)
-    kb = _k_side("fused_fp8", k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, B, NH, D, dev, q.dtype)
+    kb = _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm)
     _stage(events, "prep_end")
     _stage(events, "index_start")
-    indices, counts = _select(select, q_pool, kb, text_len, g)
+    indices, counts = _select(select, kb, text_len, g)
     _stage(events, "index_end")
     _stage(events, "attn_start")
-    _core.bsa_forward_fp8_gather(q8.flatten(2, 3), q_scale, kb["k8"].flatten(2, 3), kb["k_scale"], v_vis, kb["vt"],
-                                 g.num_txt_blk, g.T_q, g.T_k, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw, indices, counts,
-                                 1.0 / math.sqrt(D), o_out, balance=balance, sorted_lists=sorted_lists)
+    grid = (g.num_txt_blk, g.T_q, g.T_k, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw)
+    o_flat = None
+    if path == "fused":
+        _core.bsa_forward_gather(q, k_vis, v_vis, kb["kt"], kb["vt"], *grid, indices, counts, scale, o_out,
+                                 balance=balance, sorted_lists=sorted_lists)
+    elif path == "fused_fp8":
+        _core.bsa_forward_fp8_gather(kb["q_tiles"].flatten(2, 3), kb["q_scale"], kb["k8"].flatten(2, 3), kb["k_scale"],
+                                     v_vis, kb["vt"], *grid, indices, counts, scale, o_out, balance=balance,
+                                     sorted_lists=sorted_lists)
+    elif path == "tiled_fp8":
+        o_flat = _core.bsa_forward_fp8(kb["q_tiles"].flatten(2, 3), kb["q_scale"], kb["k8"].flatten(2, 3),
+                                       kb["k_scale"], kb["v_all"].flatten(2, 3), indices, counts, scale, g.bs,
+                                       balance=balance)
+    else:
+        o_flat = _core.bsa_forward(kb["q_tiles"].flatten(2, 3), kb["k_all"].flatten(2, 3), kb["v_all"].flatten(2, 3),
+                                   indices, counts, scale, g.bs, balance=balance)
     _stage(events, "attn_end")
     _stage(events, "untile_start")
+    if o_flat is not None:
+        _core.untile(o_flat.view(B, NH, g.nq_blk, g.bs, D), o_out, *grid[1:2], *grid[3:])
     _stage(events, "untile_end")
-    return o_out if o_out.dtype == out_dtype else o_out.to(out_dtype)
+    return o_out
 
 
 def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, events=None, fused=True,
@@ -319,7 +264,7 @@ def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, eve
     block (bf16 only; D = 128 and 128-token tiles, ValueError otherwise); the selection is unchanged.
     ``context`` = (ContextCache, layer key, context frames) keeps the key-side preparation of the
     fixed leading frames and the text across calls (see ContextCache).  ``normalize_k_pool`` (``select``
-    scores by cosine similarity): the fused bf16/f16 path's pool launch also writes the key pool's rows
+    scores by cosine similarity): the preparation also writes the key pool's rows
     normalised, once per key block, and the block mask takes them instead of normalising every key row in
     every workgroup of query rows (same selection, bit for bit); ``select`` then receives it as the
     keyword argument ``k_pool_normalized``.
@@ -331,38 +276,14 @@ def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, eve
             k_txt, v_txt = k_txt.to(torch.bfloat16), v_txt.to(torch.bfloat16)
     text_len = 0 if k_txt is None else k_txt.shape[2]
     g = geometry(latent_hw, tile, q.shape[2], k_vis.shape[2], text_len)
-    B, NH, _, D = q.shape
-    dev, dt = q.device, q.dtype
-    args = (q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, out_dtype, events, balance, context, sorted_lists)
-    if qk_fp8:
-        if dt != torch.bfloat16 or not fp8_supported(D, tile):
-            raise ValueError(f"qk_fp8 is built for bfloat16, D = 128 and 128-token tiles (got {dt}, D = {D}, "
-                             f"tile {tuple(tile)})")
-        if fused and uses_fused(q, k_vis, v_vis, tile, (g.H, g.W)):
-            return _fused_fp8(*args)
-        return _tiled_fp8(*args)
-    if fused and uses_fused(q, k_vis, v_vis, tile, (g.H, g.W)):
-        return _fused(*args, k_norm=normalize_k_pool)
-    _stage(events, "alloc_start")
-    q_tiled = torch.empty((B, NH, g.nq_blk, g.bs, D), device=dev, dtype=dt)
-    q_pool = torch.empty((B, NH, g.nq_blk, D), device=dev, dtype=dt)
-    _stage(events, "alloc_end")
-    _stage(events, "prep_start")
-    _core.q_prep(q, q_tiled, q_pool, g.T_q, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw)
-    kb = _k_side("tiled", k_txt, v_txt, k_vis, v_vis, g, text_len, context, B, NH, D, dev, dt)
-    _stage(events, "prep_end")
-    _stage(events, "index_start")
-    indices, counts = _select(select, q_pool, kb, text_len, g)
-    _stage(events, "index_end")
-    _stage(events, "attn_start")
-    o_flat = _core.bsa_forward(q_tiled.flatten(2, 3), kb["k_all"].flatten(2, 3), kb["v_all"].flatten(2, 3), indices,
-                               counts, 1.0 / math.sqrt(D), g.bs, balance=balance)
-    _stage(events, "attn_end")
-    _stage(events, "untile_start")
-    o_out = torch.empty_like(q)
-    _core.untile(o_flat.view(B, NH, g.nq_blk, g.bs, D), o_out, g.T_q, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw)
-    _stage(events, "untile_end")
-    return o_out if o_out.dtype == out_dtype else o_out.to(out_dtype)
+    tokens = fused and uses_fused(q, k_vis, v_vis, tile, (g.H, g.W))
+    if qk_fp8 and (q.dtype != torch.bfloat16 or not fp8_supported(q.shape[3], tile)):
+        raise ValueError(f"qk_fp8 is built for bfloat16, D = 128 and 128-token tiles (got {q.dtype}, D = {q.shape[3]}, "
+                         f"tile {tuple(tile)})")
+    path = ("fused" if tokens else "tiled") + ("_fp8" if qk_fp8 else "")
+    out = _call(path, q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, events, balance, context, sorted_lists,
+                normalize_k_pool)
+    return out if out.dtype == out_dtype else out.to(out_dtype)
 
 
 def dense_attention(q, k_txt, v_txt, k_vis, v_vis):
