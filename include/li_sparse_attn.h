@@ -200,6 +200,16 @@ int li_block_mask(int dtype, int32_t B, int32_t NH, int32_t D,
                   int32_t* indices, int32_t* counts, void* scores, void* stream);
 
 /*
+ * Range check of block ids: *flag is set to 1 when any of the n ids (device,
+ * contiguous, 16-byte aligned) lies outside [0, n_blocks) and left alone
+ * otherwise.  flag: device-accessible memory, typically a pinned host word
+ * that the caller cleared and reads once the stream has passed this call.
+ * Replaces the block_indices.max() read-back of longcat_flash_attn
+ * (HYK:194-195).
+ */
+int li_check_block_ids(const int32_t* ids, int64_t n, int32_t n_blocks, int32_t* flag, void* stream);
+
+/*
  * Block-sparse flash-attention forward.  Replaces longcat_flash_attn(q, k, v,
  * block_indices, block_counts, sm_scale, logical_block_size) and
  * _attn_fwd_bsa_align (HYK:27-155, 158-233; MG longcat_kernel.py:28-134, 137-190).

@@ -452,6 +452,34 @@ __global__ __launch_bounds__(512) void block_mask_tiled_kernel(MaskArgs a) {
   select_row<KS>(a, [&](int r) LI_MASK_INLINE { return kr[r]; }, KS, nf, qb, bh, lane);
 }
 
+// Sets *flag when any of the n ids lies outside [0, n_blocks).  One read of the
+// list, 16 ids per thread and pass; the flag (host memory) is written only when
+// an id is out of range.
+__global__ __launch_bounds__(256) void check_ids_kernel(const int32_t* ids, int64_t n, int32_t n_blocks, int32_t* flag) {
+  typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+  const uint32_t lim = (uint32_t)n_blocks;
+  const int64_t threads = (int64_t)gridDim.x * 256, me = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  bool bad = false;
+  const int64_t n4 = n >> 2;  // the list starts 16-byte aligned
+  int64_t i = me;
+  for (; i + 3 * threads < n4; i += 4 * threads) {
+    i32x4 x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = reinterpret_cast<const i32x4*>(ids)[i + k * threads];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad |= (uint32_t)x[k][e] >= lim;
+  }
+  for (; i < n4; i += threads) {
+    const i32x4 x = reinterpret_cast<const i32x4*>(ids)[i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bad |= (uint32_t)x[e] >= lim;
+  }
+  if (me < (n & 3)) bad |= (uint32_t)ids[4 * n4 + me] >= lim;
+  if (bad) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 constexpr int kTiledMaxNk = 64 * 28;
 
 // LDS bytes of the shared-pool path, or 0 when it does not apply.
@@ -531,5 +559,16 @@ extern "C" int li_block_mask(int dtype, int32_t B, int32_t NH, int32_t D, const 
   else
     return LI_ERR_UNSUPPORTED;
 #undef LI_MASK_LAUNCH
+  return launch_status();
+}
+
+extern "C" int li_check_block_ids(const int32_t* ids, int64_t n, int32_t n_blocks, int32_t* flag, void* stream) {
+  if (!ids || !flag || n < 0 || n_blocks < 0) return LI_ERR_INVALID_ARG;
+  if ((reinterpret_cast<uintptr_t>(ids) & 15u) != 0) return LI_ERR_INVALID_ARG;
+  if (n == 0) return LI_OK;
+  const int64_t wgs = (n + 4095) / 4096;
+  clear_launch_error();
+  hipLaunchKernelGGL(check_ids_kernel, dim3((unsigned)(wgs < 512 ? wgs : 512)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), ids, n, n_blocks, flag);
   return launch_status();
 }

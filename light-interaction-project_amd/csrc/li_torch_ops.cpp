@@ -451,6 +451,18 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> block_mask(const at::Tensor& q_po
   return {indices, counts, scores};
 }
 
+// Sets the pinned host word `flag` when an id of `ids` lies outside [0, n_blocks).
+void check_block_ids(const at::Tensor& ids, int64_t n_blocks, at::Tensor& flag) {
+  gpu(ids, "ids");
+  TORCH_CHECK(ids.scalar_type() == at::kInt && ids.is_contiguous(), "ids must be contiguous int32");
+  TORCH_CHECK(flag.scalar_type() == at::kInt && flag.numel() == 1 && (flag.is_cuda() || flag.is_pinned()),
+              "flag must be one int32 in pinned host or device memory");
+  TORCH_CHECK(n_blocks >= 0 && n_blocks <= INT32_MAX, "n_blocks must fit 32 bits");
+  c10::DeviceGuard guard(ids.device());
+  check("li_check_block_ids", li_check_block_ids(ids.data_ptr<int32_t>(), ids.numel(), (int32_t)n_blocks,
+                                                 flag.data_ptr<int32_t>(), stream_of(ids)));
+}
+
 void index_checks(const at::Tensor& indices, const at::Tensor& counts) {
   TORCH_CHECK(indices.scalar_type() == at::kInt && counts.scalar_type() == at::kInt,
               "block indices and counts must be int32");
@@ -743,6 +755,7 @@ TORCH_LIBRARY(li, m) {
   m.def("block_mask(Tensor q_pool, Tensor k_pool, int metric, int budget_mode, float ratio, int min_budget, "
         "int n_recent, bool force_diag, bool force_sink, bool force_neighbors, int nh, int nw, int num_txt_blk, "
         "int kmax, Tensor? row_budget, bool return_scores, bool k_normalized=False) -> (Tensor, Tensor, Tensor)");
+  m.def("check_block_ids(Tensor ids, int n_blocks, Tensor(a!) flag) -> ()");
   m.def("bsa_fwd(Tensor q, Tensor k, Tensor v, Tensor indices, Tensor counts, float sm_scale, int block_size, "
         "Tensor(a!) out, bool return_lse, bool split, bool balance) -> Tensor");
   m.def("bsa_fwd_gather(Tensor q, Tensor k, Tensor v, Tensor? k_txt, Tensor? v_txt, int num_txt_blk, int[] q_geom, "
@@ -770,6 +783,7 @@ TORCH_LIBRARY_IMPL(li, CUDA, m) {
   m.impl("kv_prep", &kv_prep);
   m.impl("untile", &untile);
   m.impl("block_mask", &block_mask);
+  m.impl("check_block_ids", &check_block_ids);
   m.impl("bsa_fwd", &bsa_fwd);
   m.impl("bsa_fwd_gather", &bsa_fwd_gather);
   m.impl("attn_dense", &attn_dense);

@@ -433,6 +433,27 @@ def block_mask(q_pool, k_pool, *, metric, budget_mode, ratio, nh, nw, num_txt_bl
     return indices, counts
 
 
+def check_block_ids(ids, n_blocks):
+    """Starts the range check of ``ids`` (contiguous int32) on the device; the returned function waits for it and says
+    whether every id lies in [0, n_blocks).  As with any read-back, not under stream capture."""
+    if ids.numel() == 0:
+        return lambda: True
+    dev = _device_check(ids)
+    with torch.cuda.device(dev):
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("block ids cannot be checked on the host while the stream is capturing")
+        flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        _run(ops.check_block_ids, ids if ids.data_ptr() % 16 == 0 else ids.clone(), n_blocks, flag)
+        done = torch.cuda.Event()
+        done.record()
+
+    def in_range():
+        done.synchronize()
+        return flag.item() == 0
+
+    return in_range
+
+
 def bsa_forward(q, k, v, indices, counts, sm_scale, block_size, return_lse=False, out=None, split=True,
                 balance=False):
     """Block-sparse attention over contiguous (B,H,L,D) tensors (see li_bsa_fwd); no host sync.

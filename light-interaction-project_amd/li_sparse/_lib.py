@@ -79,6 +79,7 @@ SIGNATURES = {
                                  ctypes.POINTER(TileGeom), _vp]),
     "li_block_mask": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _vp, _i64p, _vp, _i64p,
                                      ctypes.POINTER(MaskParams), _vp, _vp, _vp, _vp]),
+    "li_check_block_ids": (ctypes.c_int, [_vp, _i64, _i32, _vp, _vp]),
     "li_bsa_fwd": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64p, _i32,
                                   _vp, _i64p, ctypes.c_float, _i32, _vp, _vp, _vp, _i64, _i32, _vp]),
     "li_bsa_fwd_workspace_size": (ctypes.c_int64, [_i32, _i32, _i32, _i32, _i32]),

@@ -114,6 +114,11 @@ def _block_mask_fake(q_pool, k_pool, metric, budget_mode, ratio, min_budget, n_r
     return indices, counts, scores
 
 
+@torch.library.register_fake("li::check_block_ids")
+def _check_block_ids_fake(ids, n_blocks, flag):
+    return None
+
+
 @torch.library.register_fake("li::bsa_fwd")
 def _bsa_fwd_fake(q, k, v, indices, counts, sm_scale, block_size, out, return_lse, split, balance):
     B, NH, Lq, _ = q.shape

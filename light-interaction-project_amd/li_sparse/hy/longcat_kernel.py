@@ -56,7 +56,12 @@ def longcat_flash_attn(q, k, v, block_indices, block_counts, sm_scale=None, logi
     BLOCK_N = logical_block_size
     if K_len % BLOCK_N != 0:
         raise ValueError(f"K Length ({K_len}) must be divisible by logical_block_size ({BLOCK_N})")
-    if block_indices.numel() and (int(block_indices.max()) >= K_len // BLOCK_N or int(block_indices.min()) < 0):
-        raise ValueError("Sparse indices out of bounds.")
-    o = _core.bsa_forward(q, k, v, block_indices, block_counts, sm_scale, BLOCK_N)
+    in_range = _core.check_block_ids(block_indices, K_len // BLOCK_N)
+    # The kernels read nothing out of bounds for any id, so the attention is enqueued before the check's result is
+    # read: the host waits for the check alone, while the attention runs.
+    try:
+        o = _core.bsa_forward(q, k, v, block_indices, block_counts, sm_scale, BLOCK_N)
+    finally:
+        if not in_range():
+            raise ValueError("Sparse indices out of bounds.")
     return o if o.dtype == out_dtype else o.to(out_dtype)
