@@ -295,6 +295,29 @@ int li_bsa_fwd_gather(int dtype, int32_t B, int32_t NH, int32_t D,
                       void* workspace, int64_t workspace_bytes, int32_t flags, void* stream);
 
 /*
+ * li_bsa_fwd with Q read and O written in token order and K / V tiled: the
+ * tile / attend / untile sequence (HYAR:330-361) without Q tiles and untile,
+ * for the shapes and K / V views that li_bsa_fwd_gather does not take.
+ *   q (B, NH, Lq, D), out (B, NH, Lq, D): token views over q_geom, as for
+ *     li_bsa_fwd_gather; k / v (B, NH, n_key_blk, BS, D) contiguous tiles, text
+ *     blocks first
+ *   q_scale / k_scale: NULL, or the e4m3 variant (bf16, D = 128, BS = 128): q
+ *     (B, NH, nq_blk, BS, D) and k hold codes with these scales, as for
+ *     li_bsa_fwd_fp8 (q_strides unused)
+ *   lists, lse, workspace and flags as for li_bsa_fwd_gather.
+ * Same results as li_bsa_fwd (li_bsa_fwd_fp8) on the Q tiles followed by
+ * li_untile, bit for bit.  Built for BS in {64, 128} and D in {64, 128}.
+ */
+int li_bsa_fwd_qo(int dtype, int32_t B, int32_t NH, int32_t D,
+                  const void* q, const int64_t q_strides[4], const float* q_scale,
+                  const void* k, const float* k_scale, const void* v, int32_t n_key_blk,
+                  const li_tile_geom* q_geom,
+                  const int32_t* block_indices, const int64_t idx_strides[4], int32_t n_cols,
+                  const int32_t* block_counts, const int64_t cnt_strides[3],
+                  float sm_scale, void* out, const int64_t out_strides[4], float* lse,
+                  void* workspace, int64_t workspace_bytes, int32_t flags, void* stream);
+
+/*
  * li_bsa_fwd_gather without a workspace argument and without any device
  * allocation: the tail split's partials and the LI_BSA_BALANCE tile order go
  * to a scratch array of li_bsa_fwd_noalloc_scratch_bytes() bytes (32 MiB)

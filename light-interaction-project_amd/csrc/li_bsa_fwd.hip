@@ -76,7 +76,8 @@ struct Cfg {
   static constexpr int LDS_BYTES = KV_BYTES > X_BYTES ? KV_BYTES : X_BYTES;
 };
 
-template <typename E, int BS, int D>
+// G: Q and O in token order (BsaGather), K and V tiled.
+template <typename E, int BS, int D, bool G = false>
 __global__ __launch_bounds__(4 * BS) void bsa_fwd_kernel(BsaArgs a) {
   using C = Cfg<BS, D>;
   typedef typename E::vec8 vec8;
@@ -106,13 +107,23 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_kernel(BsaArgs a) {
   count = count < 0 ? 0 : (count > a.n_cols ? a.n_cols : count);
   count = __builtin_amdgcn_readfirstlane(count);
   const int row0 = m * BS;
+  // Output row of tile row rt, or null when it is not stored (past Lq, or
+  // outside the token grid).
+  auto out_row = [&](int rt) LI_INLINE -> uint16_t* {
+    if constexpr (G) {
+      bool ok;
+      const int32_t l = tile_token(a.g, a.g.Tq, m, rt, ok);
+      return ok ? a.out + b * a.g.os[0] + h * a.g.os[1] + (int64_t)l * a.g.os[2] : nullptr;
+    } else {
+      return row0 + rt < a.Lq ? ohead + (int64_t)(row0 + rt) * D : nullptr;
+    }
+  };
 
   if (count == 0) {
     // No kept block: zeros (and lse = -inf), as the reference's l_i = 1, acc = 0.
-    for (int u = tid; u < BS * (D / 8); u += C::NTHR) {
-      const int r = row0 + u / (D / 8);
-      if (r < a.Lq) *reinterpret_cast<u32x4*>(ohead + (int64_t)r * D + 8 * (u % (D / 8))) = u32x4{0u, 0u, 0u, 0u};
-    }
+    for (int u = tid; u < BS * (D / 8); u += C::NTHR)
+      if (uint16_t* orow = out_row(u / (D / 8)))
+        *reinterpret_cast<u32x4*>(orow + 8 * (u % (D / 8))) = u32x4{0u, 0u, 0u, 0u};
     if (a.lse)
       for (int r = tid; r < BS; r += C::NTHR)
         if (row0 + r < a.Lq) a.lse[(int64_t)bh * a.Lq + row0 + r] = -__builtin_inff();
@@ -122,11 +133,20 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_kernel(BsaArgs a) {
   // Q^T fragments (MFMA B operand): lane holds query row (l32) and d = 16 s + 8 hl .. +7.
   vec8 qf[C::DS];
   {
-    const int r = row0 + 32 * qq + l32;
+    const uint16_t* qrow;
+    bool ok;
+    if constexpr (G) {
+      const int32_t l = tile_token(a.g, a.g.Tq, m, 32 * qq + l32, ok);
+      qrow = a.q + b * a.g.qs[0] + h * a.g.qs[1] + (int64_t)l * a.g.qs[2];
+    } else {
+      const int r = row0 + 32 * qq + l32;
+      ok = r < a.Lq;
+      qrow = qhead + (int64_t)r * D;
+    }
 #pragma unroll
     for (int s = 0; s < C::DS; ++s) {
       u32x4 x = {0u, 0u, 0u, 0u};
-      if (r < a.Lq) x = *reinterpret_cast<const u32x4*>(qhead + (int64_t)r * D + 16 * s + 8 * hl);
+      if (ok) x = *reinterpret_cast<const u32x4*>(qrow + 16 * s + 8 * hl);
       qf[s] = __builtin_bit_cast(vec8, x);
     }
   }
@@ -338,8 +358,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_kernel(BsaArgs a) {
     const float l = lrow * a0 + l1 * a1;
     const float inv = 1.0f / l;
     const int r = row0 + 32 * qq + l32;
-    if (r < a.Lq) {
-      uint16_t* orow = ohead + (int64_t)r * D;
+    if (uint16_t* orow = out_row(32 * qq + l32)) {
 #pragma unroll
       for (int dt = 0; dt < C::NDT; ++dt)
 #pragma unroll
@@ -354,8 +373,8 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_kernel(BsaArgs a) {
           const u32x2 pk = {cvt_pk<E>(val[0], val[1]), cvt_pk<E>(val[2], val[3])};
           *reinterpret_cast<u32x2*>(orow + 32 * dt + 8 * i4 + 4 * hl) = pk;
         }
-      if (a.lse && hl == 0) a.lse[(int64_t)bh * a.Lq + r] = mm + __builtin_log2f(l);
     }
+    if (a.lse && hl == 0 && r < a.Lq) a.lse[(int64_t)bh * a.Lq + r] = mm + __builtin_log2f(l);
   }
 }
 
@@ -429,12 +448,15 @@ __device__ __forceinline__ void sched_m_phase() {
 // keeps blocks 0 .. n_cols - 1; queries and keys past the token bounds are
 // skipped, and the padding rows of the last text and visual blocks score -inf.
 // ZR (with G): the zero-region load path (BsaArgs::zero_region, gen_pairs).
-template <typename E, int BS, bool G = false, bool F8 = false, bool DN = false, bool ZR = false>
+// KT (with G): K and V tiled as without G; only Q (16-bit) and O in token order.
+template <typename E, int BS, bool G = false, bool F8 = false, bool DN = false, bool ZR = false, bool KT = false>
 __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   using C = DmaCfg<BS>;
-  static_assert(!G || BS == 128, "token-order addressing is built for 128-row tiles");
+  constexpr bool GK = G && !KT;  // K / V in token order
+  static_assert(!GK || BS == 128, "token-order K / V addressing is built for 128-row tiles");
   static_assert(!F8 || BS == 128, "the e4m3 kernel is built for 128-row blocks");
-  static_assert(!DN || (G && !F8), "dense calls use token-order addressing and 16-bit keys");
+  static_assert(!DN || (GK && !F8), "dense calls use token-order addressing and 16-bit keys");
+  static_assert(!KT || (G && !DN && !ZR), "tiled K / V with token-order Q / O");
   constexpr int D = 128;
   typedef typename E::vec8 vec8;
   typedef __attribute__((address_space(3))) void lds_void;
@@ -576,7 +598,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   // Fused path: the same granules, with the rows of a chunk one token stride
   // apart in the untiled visual K / V.
   uint32_t k_src_vis = 0, v_src_vis = 0;
-  if constexpr (G) {
+  if constexpr (GK) {
     k_src_vis = (uint32_t)(rp * a.g.ks[2] * 2) + 16u * ((lane & 15) ^ rp);
     v_src_vis = (uint32_t)(rp * a.g.vs[2] * 2) + 2u * (32 * (((lane & 15) >> 2) ^ rp) + 8 * (lane & 3));
   }
@@ -821,7 +843,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
     const char* txt_k = nullptr;
     const char* txt_v = nullptr;
     const char* zero_rows = reinterpret_cast<const char*>(g_zero_rows);
-    if constexpr (G) {
+    if constexpr (GK) {
       vis_k = reinterpret_cast<const char*>(a.k + b * a.g.ks[0] + h * a.g.ks[1]);
       vis_v = reinterpret_cast<const char*>(a.v + b * a.g.vs[0] + h * a.g.vs[1]);
       txt_k = reinterpret_cast<const char*>(a.g.ktxt + (int64_t)bh * a.g.ntxt * BS * D) + gw * LPW * 1024;
@@ -855,7 +877,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
     };
     auto geo_of = [&](int blk) LI_INLINE {
       Geo g_{blk, 0, 0u, false};
-      if constexpr (G) {
+      if constexpr (GK) {
         // Straight-line scalar code: both sides of each choice are computed;
         // the text test is skipped when there are no text blocks.
         bool txt = false;
@@ -879,10 +901,10 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
     };
     // Byte strides between K / V tokens (below 2^32: the host bounds the
     // largest row offset of a tile).
-    const uint32_t kst = G ? (uint32_t)(2 * a.g.ks[2]) : 0u, vst = G ? (uint32_t)(2 * a.g.vs[2]) : 0u;
+    const uint32_t kst = GK ? (uint32_t)(2 * a.g.ks[2]) : 0u, vst = GK ? (uint32_t)(2 * a.g.vs[2]) : 0u;
     auto blk_src = [&](const Geo& g_, bool is_v) LI_INLINE {
       Blk s_{nullptr, nullptr, 0u};
-      if constexpr (!G) {
+      if constexpr (!GK) {
         s_.alt = is_v ? reinterpret_cast<const char*>(vhead + (int64_t)g_.blk * BS * D) + gw * LPW * 1024
                       : kbytes + (int64_t)g_.blk * BS * D * KEB + gw * KPW * 1024;
       } else {
@@ -909,7 +931,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
       const Blk& s_ = isv ? sv : sk;
       const uint32_t lin = isv ? v_src : (F8 ? k8_src[j & 1] : k_src);
       const char* alt = j < 4 ? s_.alt : s_.alt + 4096;
-      if (!G || (F8 && !isv))
+      if (!GK || (F8 && !isv))
         return DmaSrc{alt, lin};
       else if constexpr (decltype(zr)::value == 1)
         return dma_sel_base(s_.mask, j, s_.vis, a.zero_region, isv ? vvo[j] : kvo[j]);
@@ -1379,10 +1401,14 @@ int launch_bsa_gather(BsaArgs& a, hipStream_t s) {
   return launch_status();
 }
 
-template <bool G>
+// KT: V tiled, O in token order (with G).
+template <bool G, bool KT = false>
 int launch_bsa_fp8(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
-  if (G && a.zero_region)
+  if constexpr (KT)
+    hipLaunchKernelGGL((bsa_fwd_dma_kernel<Bf16, 128, true, true, false, false, true>), dim3(attn_units(a)),
+                       dim3(DmaCfg<128>::NTHR), 0, s, a);
+  else if (G && a.zero_region)
     hipLaunchKernelGGL((bsa_fwd_dma_kernel<Bf16, 128, G, true, false, G>), dim3(attn_units(a)),
                        dim3(DmaCfg<128>::NTHR), 0, s, a);
   else
@@ -1392,27 +1418,28 @@ int launch_bsa_fp8(BsaArgs& a, hipStream_t s) {
   return launch_status();
 }
 
-template <typename E, int BS>
+// QO: token-order Q and O (BsaArgs::g) with tiled K and V.
+template <typename E, int BS, bool QO>
 int launch_bsa_dma(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
-  hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, BS>), dim3(attn_units(a)), dim3(DmaCfg<BS>::NTHR), 0, s, a);
-  if constexpr (BS == 128) launch_merge<E, false>(a, s);
+  hipLaunchKernelGGL((bsa_fwd_dma_kernel<E, BS, QO, false, false, false, QO>), dim3(attn_units(a)), dim3(DmaCfg<BS>::NTHR), 0, s, a);
+  if constexpr (BS == 128) launch_merge<E, QO>(a, s);
   return launch_status();
 }
 
-template <typename E, int BS, int D>
+template <typename E, int BS, int D, bool QO>
 int launch_bsa(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
-  hipLaunchKernelGGL((bsa_fwd_kernel<E, BS, D>), dim3(a.ntiles), dim3(Cfg<BS, D>::NTHR), 0, s, a);
+  hipLaunchKernelGGL((bsa_fwd_kernel<E, BS, D, QO>), dim3(a.ntiles), dim3(Cfg<BS, D>::NTHR), 0, s, a);
   return launch_status();
 }
 
-template <typename E>
+template <typename E, bool QO>
 int dispatch_bsa(BsaArgs& a, int bs, int D, hipStream_t s) {
-  if (bs == 128 && D == 128) return launch_bsa_dma<E, 128>(a, s);
-  if (bs == 128 && D == 64) return launch_bsa<E, 128, 64>(a, s);
-  if (bs == 64 && D == 128) return launch_bsa_dma<E, 64>(a, s);
-  if (bs == 64 && D == 64) return launch_bsa<E, 64, 64>(a, s);
+  if (bs == 128 && D == 128) return launch_bsa_dma<E, 128, QO>(a, s);
+  if (bs == 128 && D == 64) return launch_bsa<E, 128, 64, QO>(a, s);
+  if (bs == 64 && D == 128) return launch_bsa_dma<E, 64, QO>(a, s);
+  if (bs == 64 && D == 64) return launch_bsa<E, 64, 64, QO>(a, s);
   return LI_ERR_UNSUPPORTED;
 }
 
@@ -1648,8 +1675,8 @@ extern "C" int li_bsa_fwd(int dtype, int32_t B, int32_t NH, int32_t Lq, int32_t 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int st = plan_units(a, tiles, D, block_size, workspace, workspace_bytes, flags, s);
   if (st != LI_OK) return st;
-  if (dtype == LI_DTYPE_BF16) return dispatch_bsa<Bf16>(a, block_size, D, s);
-  return dispatch_bsa<F16>(a, block_size, D, s);
+  if (dtype == LI_DTYPE_BF16) return dispatch_bsa<Bf16, false>(a, block_size, D, s);
+  return dispatch_bsa<F16, false>(a, block_size, D, s);
 }
 
 namespace {
@@ -1702,6 +1729,27 @@ void setup_zero_region(BsaArgs& a, int64_t max_row, int64_t st, int32_t ntxt) {
   a.gen_pairs = ((ntxt > 1 ? ntxt - 1 : 0) + 1) & ~1;
 }
 
+
+// The tile grid of the queries.
+void set_grid(BsaGather& g, const li_tile_geom& gq) {
+  g.H = gq.H;
+  g.W = gq.W;
+  g.tt = gq.tt;
+  g.th = gq.th;
+  g.tw = gq.tw;
+  g.nh = gq.nh;
+  g.nw = gq.nw;
+  g.Tq = gq.T;
+  g.mg_nhnw = magic16(gq.nh * gq.nw);
+  g.mg_nw = magic16(gq.nw);
+  g.mg_thtw = magic16(gq.th * gq.tw);
+  g.mg_tw = magic16(gq.tw);
+  g.id_nhnw = gq.nh * gq.nw == 1 ? ~0u : 0u;
+  g.id_nw = gq.nw == 1 ? ~0u : 0u;
+  g.q_tokens = gq.T * gq.H * gq.W;
+  g.txt_tail = 0;
+  g.vis_tail = 0;
+}
 
 // Checks and BsaArgs of a token-order (fused) call over the q_geom / k_geom
 // grids.  With e4m3 keys (k8) only V is read in token order: k / k_strides
@@ -1770,6 +1818,7 @@ int gather_setup(BsaArgs& a, int64_t& tiles, int32_t B, int32_t NH, int32_t D, c
   a.n_cols = n_cols;
   a.qk_scale = sm_scale * 1.44269504f;
   BsaGather& g = a.g;
+  set_grid(g, gq);
   for (int i = 0; i < 3; ++i) {
     g.qs[i] = k8 ? 0 : q_strides[i];
     g.ks[i] = k8 ? v_strides[i] : k_strides[i];
@@ -1779,25 +1828,8 @@ int gather_setup(BsaArgs& a, int64_t& tiles, int32_t B, int32_t NH, int32_t D, c
   g.ktxt = static_cast<const uint16_t*>(k_txt);
   g.vtxt = static_cast<const uint16_t*>(v_txt);
   g.ntxt = num_txt_blk;
-  g.H = gq.H;
-  g.W = gq.W;
-  g.tt = gq.tt;
-  g.th = gq.th;
-  g.tw = gq.tw;
-  g.nh = gq.nh;
-  g.nw = gq.nw;
-  g.Tq = gq.T;
   g.Tk = gk.T;
-  g.mg_nhnw = magic16(gq.nh * gq.nw);
-  g.mg_nw = magic16(gq.nw);
-  g.mg_thtw = magic16(gq.th * gq.tw);
-  g.mg_tw = magic16(gq.tw);
-  g.id_nhnw = gq.nh * gq.nw == 1 ? ~0u : 0u;
-  g.id_nw = gq.nw == 1 ? ~0u : 0u;
-  g.q_tokens = gq.T * gq.H * gq.W;
   g.k_tokens = gk.T * gk.H * gk.W;
-  g.txt_tail = 0;
-  g.vis_tail = 0;
   return LI_OK;
 }
 
@@ -1823,6 +1855,64 @@ extern "C" int li_bsa_fwd_gather(int dtype, int32_t B, int32_t NH, int32_t D, co
   if (st != LI_OK) return st;
   if (dtype == LI_DTYPE_BF16) return launch_bsa_gather<Bf16>(a, s);
   return launch_bsa_gather<F16>(a, s);
+}
+
+extern "C" int li_bsa_fwd_qo(int dtype, int32_t B, int32_t NH, int32_t D, const void* q, const int64_t q_strides[4],
+                             const float* q_scale, const void* k, const float* k_scale, const void* v,
+                             int32_t n_key_blk, const li_tile_geom* q_geom, const int32_t* block_indices,
+                             const int64_t idx_strides[4], int32_t n_cols, const int32_t* block_counts,
+                             const int64_t cnt_strides[3], float sm_scale, void* out, const int64_t out_strides[4],
+                             float* lse, void* workspace, int64_t workspace_bytes, int32_t flags, void* stream) {
+  const bool fp8 = q_scale != nullptr;
+  if (!q || !k || !v || !q_geom || !block_indices || !idx_strides || !block_counts || !cnt_strides || !out_strides ||
+      (!fp8 && !q_strides) || fp8 != (k_scale != nullptr))
+    return LI_ERR_INVALID_ARG;
+  if (B <= 0 || NH <= 0 || n_cols < 0 || n_key_blk < 0) return LI_ERR_INVALID_ARG;
+  if (dtype != LI_DTYPE_BF16 && dtype != LI_DTYPE_F16) return LI_ERR_UNSUPPORTED;
+  const li_tile_geom& gq = *q_geom;
+  if (gq.H <= 0 || gq.W <= 0 || gq.tt <= 0 || gq.th <= 0 || gq.tw <= 0 || gq.T < 0) return LI_ERR_SHAPE;
+  if (gq.nh != (gq.H + gq.th - 1) / gq.th || gq.nw != (gq.W + gq.tw - 1) / gq.tw) return LI_ERR_SHAPE;
+  const int64_t bs = (int64_t)gq.tt * gq.th * gq.tw;
+  if (!(bs == 64 || bs == 128) || !(D == 64 || D == 128)) return LI_ERR_UNSUPPORTED;
+  if (fp8 && (dtype != LI_DTYPE_BF16 || D != 128 || bs != 128)) return LI_ERR_UNSUPPORTED;
+  if (fp8 ? !aligned16(q) : !row_view_ok(q, q_strides)) return LI_ERR_INVALID_ARG;
+  if (!row_view_ok(out, out_strides) || !aligned16(k) || !aligned16(v)) return LI_ERR_INVALID_ARG;
+  const int64_t nq = (int64_t)((gq.T + gq.tt - 1) / gq.tt) * gq.nh * gq.nw;
+  if ((int64_t)gq.nh * gq.nw >= 65536 || nq >= 65536) return LI_ERR_SHAPE;
+  if ((int64_t)gq.T * gq.H * gq.W >= (1ll << 31)) return LI_ERR_SHAPE;
+  if (n_key_blk == 0) return LI_ERR_SHAPE;  // no key block at all
+  if (nq == 0) return LI_OK;
+  const int64_t tiles = nq * B * NH;
+  if (tiles > 0x7FFFFFFF) return LI_ERR_SHAPE;
+  BsaArgs a = {};
+  a.q = static_cast<const uint16_t*>(q);
+  a.k = static_cast<const uint16_t*>(k);
+  a.v = static_cast<const uint16_t*>(v);
+  a.q_scale = q_scale;
+  a.k_scale = k_scale;
+  a.idx = block_indices;
+  for (int i = 0; i < 4; ++i) a.is[i] = idx_strides[i];
+  a.cnt = block_counts;
+  for (int i = 0; i < 3; ++i) a.cs[i] = cnt_strides[i];
+  a.out = static_cast<uint16_t*>(out);
+  a.lse = lse;
+  a.NH = NH;
+  a.Lq = (int32_t)(nq * bs);
+  a.nkb = n_key_blk;
+  a.nqt = (int32_t)nq;
+  a.n_cols = n_cols;
+  a.qk_scale = sm_scale * 1.44269504f;
+  set_grid(a.g, gq);
+  for (int i = 0; i < 3; ++i) {
+    a.g.qs[i] = fp8 ? 0 : q_strides[i];
+    a.g.os[i] = out_strides[i];
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int st = plan_units(a, tiles, D, (int32_t)bs, workspace, workspace_bytes, flags, s);
+  if (st != LI_OK) return st;
+  if (fp8) return launch_bsa_fp8<true, true>(a, s);
+  if (dtype == LI_DTYPE_BF16) return dispatch_bsa<Bf16, true>(a, (int)bs, D, s);
+  return dispatch_bsa<F16, true>(a, (int)bs, D, s);
 }
 
 // Scratch of li_bsa_fwd_gather_noalloc: the tail split's partials or the

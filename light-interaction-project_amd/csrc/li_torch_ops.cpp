@@ -545,6 +545,59 @@ at::Tensor bsa_fwd_gather(const at::Tensor& q, const at::Tensor& k, const at::Te
   return lse;
 }
 
+// q: a 16-bit token view, or with scales e4m3 tiles (B, NH, nq, BS, D); k, v: contiguous (B, NH, blocks, BS, D) tiles.
+at::Tensor bsa_fwd_qo(const at::Tensor& q, const OptTensor& q_scale, const at::Tensor& k, const OptTensor& k_scale,
+                      const at::Tensor& v, c10::IntArrayRef q_geom, const at::Tensor& indices,
+                      const at::Tensor& counts, double sm_scale, at::Tensor& out, bool return_lse, bool split,
+                      bool balance) {
+  gpu(q, "q");
+  rank(out, 4, "out");
+  index_checks(indices, counts);
+  c10::DeviceGuard guard(q.device());
+  const li_tile_geom gq = geom_of(q_geom);
+  const int64_t B = out.size(0), NH = out.size(1), D = out.size(3), nq = blocks_of(gq), bs = block_size_of(gq);
+  const bool fp8 = given(q_scale);
+  TORCH_CHECK(fp8 == given(k_scale), "q_scale and k_scale go together");
+  rank(k, 5, "k");
+  const int64_t nk = k.size(2);
+  TORCH_CHECK(k.is_contiguous() && v.is_contiguous(), "k and v tiles must be contiguous");
+  TORCH_CHECK(v.sizes() == k.sizes(), "v must have k's shape ", k.sizes(), ", got ", v.sizes());
+  tiles5(k, B, NH, nk, bs, D, "k", q);
+  tiles5(v, B, NH, nk, bs, D, "v", q);
+  rows4(out, B, NH, tokens_of(gq), D, "out", &v);
+  std::array<int64_t, 4> qs{};
+  if (fp8) {
+    TORCH_CHECK(q.is_contiguous() && q.dim() == 5 && q.size(2) == nq && q_scale->is_contiguous() &&
+                    k_scale->is_contiguous(),
+                "q tiles and the scales must be contiguous, q of ", nq, " tiles");
+    tiles5(q, B, NH, nq, bs, D, "q", q);
+    codes(q, "q");
+    codes(k, "k");
+    scales3(*q_scale, B, NH, nq, "q_scale", q, true);
+    scales3(*k_scale, B, NH, nk, "k_scale", q, true);
+  } else {
+    rank(q, 4, "q");
+    rows4(q, B, NH, tokens_of(gq), D, "q", &v);
+    TORCH_CHECK(k.scalar_type() == v.scalar_type(), "k must be ", v.scalar_type());
+    qs = strides<4>(q);
+  }
+  lists(indices, counts, B, NH, nq, q);
+  at::Tensor lse = lse_or_empty(v, return_lse, B, NH, nq * bs);
+  at::Tensor ws = workspace(v, B, NH, nq * bs, D, bs, indices.size(3), split || balance);
+  const auto os = strides<4>(out);
+  const auto is = strides<4>(indices);
+  const auto cs = strides<3>(counts);
+  check("li_bsa_fwd_qo",
+        li_bsa_fwd_qo(dtype_code(v), (int32_t)B, (int32_t)NH, (int32_t)D, q.data_ptr(), fp8 ? nullptr : qs.data(),
+                      fp8 ? q_scale->data_ptr<float>() : nullptr, k.data_ptr(),
+                      fp8 ? k_scale->data_ptr<float>() : nullptr, v.data_ptr(), (int32_t)nk, &gq,
+                      indices.data_ptr<int32_t>(), is.data(), (int32_t)indices.size(3), counts.data_ptr<int32_t>(),
+                      cs.data(), (float)sm_scale, out.data_ptr(), os.data(),
+                      return_lse ? lse.data_ptr<float>() : nullptr, ptr(ws), ws.defined() ? ws.numel() * 4 : 0,
+                      balance ? LI_BSA_BALANCE : 0, stream_of(q)));
+  return lse;
+}
+
 at::Tensor attn_dense(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                       const c10::optional<at::Tensor>& k_txt, const c10::optional<at::Tensor>& v_txt,
                       int64_t txt_len, double sm_scale, at::Tensor& out, bool return_lse, bool split) {
@@ -761,6 +814,8 @@ TORCH_LIBRARY(li, m) {
   m.def("bsa_fwd_gather(Tensor q, Tensor k, Tensor v, Tensor? k_txt, Tensor? v_txt, int num_txt_blk, int[] q_geom, "
         "int[] k_geom, Tensor indices, Tensor counts, float sm_scale, Tensor(a!) out, bool return_lse, bool split, "
         "bool balance, bool sorted=False) -> Tensor");
+  m.def("bsa_fwd_qo(Tensor q, Tensor? q_scale, Tensor k, Tensor? k_scale, Tensor v, int[] q_geom, Tensor indices, "
+        "Tensor counts, float sm_scale, Tensor(a!) out, bool return_lse, bool split, bool balance) -> Tensor");
   m.def("attn_dense(Tensor q, Tensor k, Tensor v, Tensor? k_txt, Tensor? v_txt, int txt_len, float sm_scale, "
         "Tensor(a!) out, bool return_lse, bool split) -> Tensor");
   m.def("tile_prep_fp8(Tensor src, Tensor(a!) dst, Tensor(b!) scales, Tensor(c!)? mean, int dst_off, int pool_off, "
@@ -786,6 +841,7 @@ TORCH_LIBRARY_IMPL(li, CUDA, m) {
   m.impl("check_block_ids", &check_block_ids);
   m.impl("bsa_fwd", &bsa_fwd);
   m.impl("bsa_fwd_gather", &bsa_fwd_gather);
+  m.impl("bsa_fwd_qo", &bsa_fwd_qo);
   m.impl("attn_dense", &attn_dense);
   m.impl("tile_prep_fp8", &tile_prep_fp8);
   m.impl("kv_prep_fp8", &kv_prep_fp8);

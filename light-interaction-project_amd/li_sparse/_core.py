@@ -559,6 +559,20 @@ def bsa_forward_fp8_gather(q8, q_scale, k8, k_scale, v, v_txt, num_txt_blk, T_q,
     return (out, lse) if return_lse else out
 
 
+def bsa_forward_qo(q, k, v, geom_q, indices, counts, sm_scale, out, *, q_scale=None, k_scale=None, return_lse=False,
+                   split=True, balance=False):
+    """Block-sparse attention with Q read and ``out`` written in token order over ``geom_q`` and K / V as contiguous
+    (B, NH, blocks, BS, D) tiles (see li_bsa_fwd_qo); with scales, q and k are e4m3 tiles.  No host sync."""
+    _device_check(q, k, v, out, indices, counts)
+    if q_scale is None:
+        _same_dtype(q, k, v, out)
+    if indices.dtype != torch.int32 or counts.dtype != torch.int32:
+        raise TypeError("block indices and counts must be int32")
+    lse = _run(ops.bsa_fwd_qo, q, q_scale, k, k_scale, v, geom_q, indices, counts, float(sm_scale), out,
+               bool(return_lse), bool(split), bool(balance))
+    return (out, lse) if return_lse else out
+
+
 def dense_supported(q, k, v, k_txt=None):
     """Inputs li_attn_fwd_dense takes: fp16/bf16, D = 128, Lk a multiple of 4, token views with unit d stride,
     8-element-multiple strides, 16-byte aligned, K/V token strides >= D."""

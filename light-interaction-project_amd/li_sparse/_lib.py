@@ -91,6 +91,9 @@ SIGNATURES = {
                                                  _vp, _vp, _i32, ctypes.POINTER(TileGeom), ctypes.POINTER(TileGeom),
                                                  _vp, _i64p, _i32, _vp, _i64p, ctypes.c_float, _vp, _i64p, _vp, _i32,
                                                  _vp]),
+    "li_bsa_fwd_qo": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _vp, _i64p, _vp, _vp, _vp, _vp, _i32,
+                                     ctypes.POINTER(TileGeom), _vp, _i64p, _i32, _vp, _i64p, ctypes.c_float, _vp,
+                                     _i64p, _vp, _vp, _i64, _i32, _vp]),
     "li_bsa_fwd_noalloc_scratch_bytes": (ctypes.c_int64, []),
     "li_tile_prep_fp8": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
                                         _i64, _i64, ctypes.POINTER(TileGeom), _vp]),

@@ -135,6 +135,12 @@ def _bsa_fwd_gather_fake(q, k, v, k_txt, v_txt, num_txt_blk, q_geom, k_geom, ind
     return _lse(q, return_lse, B, NH, _nblk(q_geom) * bs)
 
 
+@torch.library.register_fake("li::bsa_fwd_qo")
+def _bsa_fwd_qo_fake(q, q_scale, k, k_scale, v, q_geom, indices, counts, sm_scale, out, return_lse, split, balance):
+    B, NH = out.shape[:2]
+    return _lse(v, return_lse, B, NH, _nblk(q_geom) * q_geom[3] * q_geom[4] * q_geom[5])
+
+
 @torch.library.register_fake("li::attn_dense")
 def _attn_dense_fake(q, k, v, k_txt, v_txt, txt_len, sm_scale, out, return_lse, split):
     B, NH, Lq, _ = q.shape

@@ -68,6 +68,15 @@ def _fusable(*ts):
     return True
 
 
+def _token_rows(*ts):
+    """Token views whose rows the tiled-K/V kernels read (Q) and write (O): unit d stride, 16-byte aligned rows."""
+    for t in ts:
+        st = t.stride()
+        if st[3] != 1 or any(x % 8 for x in st[:3]) or st[2] <= 0 or t.data_ptr() % 16:
+            return False
+    return True
+
+
 def uses_fused(q, k_vis, v_vis, tile, latent_hw):
     """True when ``sparse_attention(..., fused=True)`` takes the fused kernel for these inputs."""
     return _core.fused_supported(q.shape[3], tile, latent_hw) and _fusable(q, k_vis, v_vis)
@@ -129,15 +138,15 @@ def context_of(sparse_params, block_idx):
 def _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm):
     """What one call prepares of its tensors, in one launch (li_prep): a dict of the buffers.
 
-    path: "fused" (pools; padded text K/V), "fused_fp8" (e4m3 Q and K tiles + scales, pools; padded text V), "tiled"
-    (Q, K, V tiles, pools), "tiled_fp8" (e4m3 Q and K tiles + scales, V tiles, pools).  Query-side buffers are the
-    call's own; key-side ones (text blocks, then the visual blocks from the first uncached frame) are the
+    path: "fused" (pools; padded text K/V), "fused_fp8" (e4m3 Q and K tiles + scales, pools; padded text V), "mixed"
+    (K, V tiles, pools), "tiled" (Q, K, V tiles, pools), "mixed_fp8" and "tiled_fp8" (e4m3 Q and K tiles + scales, V
+    tiles, pools).  Query-side buffers are the call's own; key-side ones (text blocks, then the visual blocks from the first uncached frame) are the
     ContextCache's where there is one.  k_norm: also keep the K pool's rows normalised for the cosine selection
     (``k_pool_n``; the selection takes it as ``k_pool_normalized``).
     """
     B, NH, _, D = q.shape
     dt = q.dtype
-    fp8, tiled = path in ("fused_fp8", "tiled_fp8"), path in ("tiled", "tiled_fp8")
+    fp8, tiled = path.endswith("_fp8"), not path.startswith("fused")
     if path == "fused" and text_len > 0:
         _core._same_dtype(q, k_txt, v_txt)
     elif text_len > 0:
@@ -157,7 +166,7 @@ def _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm):
         if fp8:
             bufs["k8"] = q.new_empty((B, NH, nkb, g.bs, D), dtype=_core.FP8)
             bufs["k_scale"] = q.new_empty((B, NH, nkb), dtype=torch.float32)
-        if path == "tiled":
+        elif tiled:
             bufs["k_all"] = q.new_empty((B, NH, nkb, g.bs, D))
         if tiled:
             bufs["v_all"] = q.new_empty((B, NH, nkb, g.bs, D))
@@ -175,7 +184,7 @@ def _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm):
     if fp8:
         out["q_tiles"] = q.new_empty((B, NH, g.nq_blk, g.bs, D), dtype=_core.FP8)
         out["q_scale"] = q.new_empty((B, NH, g.nq_blk), dtype=torch.float32)
-    elif tiled:
+    elif path == "tiled":
         out["q_tiles"] = q.new_empty((B, NH, g.nq_blk, g.bs, D))
     if first > 0:
         k_vis, v_vis = k_vis[:, :, first * g.H * g.W:], v_vis[:, :, first * g.H * g.W:]
@@ -207,13 +216,10 @@ def fp8_supported(D, tile):
     return D == 128 and tile[0] * tile[1] * tile[2] == 128
 
 
-def _call(path, q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, events, balance, ctx, sorted_lists, k_norm):
-    """Preparation, block selection, attention, and the untile of the tiled paths."""
+def _call(path, q, k_txt, v_txt, k_vis, v_vis, o_out, g, select, text_len, events, balance, ctx, sorted_lists, k_norm):
+    """Preparation, block selection, attention into ``o_out``, and the untile of the tiled paths."""
     B, NH, _, D = q.shape
     scale = 1.0 / math.sqrt(D)
-    _stage(events, "alloc_start")
-    o_out = torch.empty_like(q)
-    _stage(events, "alloc_end")
     _stage(events, "prep_start")
     kb = _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm)
     _stage(events, "prep_end")
@@ -230,6 +236,11 @@ def _call(path, q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, events, bala
         _core.bsa_forward_fp8_gather(kb["q_tiles"].flatten(2, 3), kb["q_scale"], kb["k8"].flatten(2, 3), kb["k_scale"],
                                      v_vis, kb["vt"], *grid, indices, counts, scale, o_out, balance=balance,
                                      sorted_lists=sorted_lists)
+    elif path.startswith("mixed"):
+        fp8 = path == "mixed_fp8"
+        _core.bsa_forward_qo(kb["q_tiles"] if fp8 else q, kb["k8"] if fp8 else kb["k_all"], kb["v_all"],
+                             (g.T_q, g.H, g.W, g.tt, g.th, g.tw, g.nh, g.nw), indices, counts, scale, o_out,
+                             q_scale=kb["q_scale"], k_scale=kb["k_scale"], balance=balance)
     elif path == "tiled_fp8":
         o_flat = _core.bsa_forward_fp8(kb["q_tiles"].flatten(2, 3), kb["q_scale"], kb["k8"].flatten(2, 3),
                                        kb["k_scale"], kb["v_all"].flatten(2, 3), indices, counts, scale, g.bs,
@@ -242,7 +253,6 @@ def _call(path, q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, events, bala
     if o_flat is not None:
         _core.untile(o_flat.view(B, NH, g.nq_blk, g.bs, D), o_out, *grid[1:2], *grid[3:])
     _stage(events, "untile_end")
-    return o_out
 
 
 def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, events=None, fused=True,
@@ -258,8 +268,8 @@ def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, eve
     ``fused`` (default) runs pools + one gather/attend/untile kernel where the
     shape allows it (D = 128, 128-token tiles, tw and W multiples of 4, a grid
     at least one tile high and wide, token views with unit d stride);
-    otherwise, or with ``fused=False``, the tiled sequence q_prep / kv_prep /
-    attention / untile.  Both give the same bits.  ``balance`` (rows with their own budgets) starts
+    otherwise, or with ``fused=False``, K and V are tiled first and the kernel reads Q and writes O in
+    token order (or Q is tiled and O untiled too, for views it cannot read).  All give the same bits.  ``balance`` (rows with their own budgets) starts
     the longest query tiles first.  ``qk_fp8`` takes Q K^T on e4m3 codes with one scale per tile
     block (bf16 only; D = 128 and 128-token tiles, ValueError otherwise); the selection is unchanged.
     ``context`` = (ContextCache, layer key, context frames) keeps the key-side preparation of the
@@ -280,9 +290,15 @@ def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, eve
     if qk_fp8 and (q.dtype != torch.bfloat16 or not fp8_supported(q.shape[3], tile)):
         raise ValueError(f"qk_fp8 is built for bfloat16, D = 128 and 128-token tiles (got {q.dtype}, D = {q.shape[3]}, "
                          f"tile {tuple(tile)})")
-    path = ("fused" if tokens else "tiled") + ("_fp8" if qk_fp8 else "")
-    out = _call(path, q, k_txt, v_txt, k_vis, v_vis, g, select, text_len, events, balance, context, sorted_lists,
-                normalize_k_pool)
+    # Q and O in token order wherever their rows can be read and written: the tiles of Q and the untile pass are for
+    # other views and for grids past the kernel's 16-bit block numbers.
+    _stage(events, "alloc_start")
+    out = torch.empty_like(q)
+    _stage(events, "alloc_end")
+    rows = g.nq_blk < 65536 and (_token_rows(out) if qk_fp8 else _token_rows(q, out))
+    path = ("fused" if tokens else "mixed" if rows else "tiled") + ("_fp8" if qk_fp8 else "")
+    _call(path, q, k_txt, v_txt, k_vis, v_vis, out, g, select, text_len, events, balance, context, sorted_lists,
+          normalize_k_pool)
     return out if out.dtype == out_dtype else out.to(out_dtype)
 
 
