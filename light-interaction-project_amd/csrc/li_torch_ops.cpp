@@ -790,6 +790,87 @@ at::Tensor bsa_fwd_fp8_gather(const at::Tensor& q8, const at::Tensor& q_scale, c
   return lse;
 }
 
+// (B, H, L, D) rows that the kernels read and write 16 bytes at a time; `apart`:
+// that also do not overlap, as the token-order K / V loads need.
+bool token_rows(const at::Tensor& t, bool apart) {
+  return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 &&
+         (apart ? t.stride(2) >= t.size(3) : t.stride(2) > 0) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+// One whole sparse-attention call into `out`: preparation, block selection and
+// attention (and the untile of query views whose rows cannot be read), the same
+// launches as the operators above one by one.  geom = (H, W, tt, th, tw); mask =
+// (metric, budget_mode, min_budget, n_recent, diag, sink, neighbors, kmax).
+void sparse_call(const at::Tensor& q, const OptTensor& k_txt, const OptTensor& v_txt, const at::Tensor& k,
+                 const at::Tensor& v, c10::IntArrayRef geom, c10::IntArrayRef mask, double ratio,
+                 const OptTensor& row_budget, bool fp8, bool k_norm, bool balance, at::Tensor& out) {
+  gpu(q, "q");
+  rank(q, 4, "q");
+  rank(k, 4, "k");
+  rank(v, 4, "v");
+  TORCH_CHECK(geom.size() == 5 && mask.size() == 8, "geom is (H, W, tt, th, tw), mask has 8 entries");
+  for (const int64_t x : geom) TORCH_CHECK(x > 0, "geom must be positive, got ", geom);
+  c10::DeviceGuard guard(q.device());
+  const int64_t B = q.size(0), NH = q.size(1), D = q.size(3);
+  const int64_t H = geom[0], W = geom[1], tt = geom[2], th = geom[3], tw = geom[4], bs = tt * th * tw;
+  const int64_t nh = (H + th - 1) / th, nw = (W + tw - 1) / tw, Tq = q.size(2) / (H * W), Tk = k.size(2) / (H * W);
+  const int64_t nq = (Tq + tt - 1) / tt * nh * nw, nk = (Tk + tt - 1) / tt * nh * nw;
+  const int64_t text_len = given(k_txt) ? k_txt->size(2) : 0, ntxt = (text_len + bs - 1) / bs;
+  const std::array<int64_t, 8> gq{Tq, H, W, tt, th, tw, nh, nw}, gk{Tk, H, W, tt, th, tw, nh, nw};
+  const bool tokens = D == 128 && bs == 128 && tw % 4 == 0 && W % 4 == 0 && H >= th && W >= tw &&
+                      token_rows(q, true) && token_rows(k, true) && token_rows(v, true);
+  const bool rows = nq < 65536 && token_rows(out, false) && (fp8 || token_rows(q, false));
+  const auto o16 = q.options(), o8 = o16.dtype(at::kFloat8_e4m3fn), o32 = o16.dtype(at::kFloat);
+  at::Tensor q_pool = at::empty({B, NH, nq, D}, o16), k_pool = at::empty({B, NH, nk, D}, o16);
+  OptTensor k_pool_n, q_tiles, q_scale, k_tiles, k_scale, v_tiles, kt, vt, txt_k, txt_v;
+  if (k_norm) k_pool_n = at::empty({B, NH, nk, D}, o16);
+  if (fp8) {
+    q_tiles = at::empty({B, NH, nq, bs, D}, o8);
+    q_scale = at::empty({B, NH, nq}, o32);
+    k_tiles = at::empty({B, NH, ntxt + nk, bs, D}, o8);
+    k_scale = at::empty({B, NH, ntxt + nk}, o32);
+  } else if (!tokens) {
+    if (!rows) q_tiles = at::empty({B, NH, nq, bs, D}, o16);
+    k_tiles = at::empty({B, NH, ntxt + nk, bs, D}, o16);
+  }
+  if (!tokens) v_tiles = at::empty({B, NH, ntxt + nk, bs, D}, o16);
+  if (text_len > 0 && tokens) {
+    // Whole blocks of text are read where they are.
+    const bool whole = text_len % bs == 0;
+    auto text_rows = [&](const at::Tensor& t, OptTensor& use, OptTensor& write) {
+      use = whole && t.is_contiguous() ? t : at::empty({B, NH, ntxt * bs, D}, o16);
+      if (!(whole && t.is_contiguous())) write = use;
+    };
+    TORCH_CHECK(given(v_txt), "v_txt must have k_txt's shape");
+    if (!fp8) text_rows(*k_txt, kt, txt_k);
+    text_rows(*v_txt, vt, txt_v);
+  }
+  prep(q, q_tiles, q_scale, q_pool, gq, k, v, k_tiles, k_scale, v_tiles, k_pool, k_pool_n, 0, gk, ntxt, k_txt, v_txt,
+       txt_k, txt_v);
+  const auto sel = block_mask(q_pool, k_norm ? *k_pool_n : k_pool, mask[0], mask[1], ratio, mask[2], mask[3], mask[4],
+                              mask[5], mask[6], nh, nw, ntxt, mask[7], row_budget, false, k_norm);
+  const at::Tensor& ind = std::get<0>(sel);
+  const at::Tensor& cnt = std::get<1>(sel);
+  const double scale = 1.0 / std::sqrt((double)D);
+  if (tokens && fp8) {
+    bsa_fwd_fp8_gather(q_tiles->flatten(2, 3), *q_scale, k_tiles->flatten(2, 3), *k_scale, v, vt, ntxt, gq, gk, ind, cnt,
+                       scale, out, false, balance, true);
+  } else if (tokens) {
+    bsa_fwd_gather(q, k, v, kt, vt, ntxt, gq, gk, ind, cnt, scale, out, false, true, balance, true);
+  } else if (rows) {
+    bsa_fwd_qo(fp8 ? *q_tiles : q, q_scale, *k_tiles, k_scale, *v_tiles, gq, ind, cnt, scale, out, false, true, balance);
+  } else {
+    at::Tensor o = at::empty({B, NH, nq * bs, D}, o16);
+    if (fp8)
+      bsa_fwd_fp8(q_tiles->flatten(2, 3), *q_scale, k_tiles->flatten(2, 3), *k_scale, v_tiles->flatten(2, 3), ind, cnt,
+                  scale, bs, o, false, true, balance);
+    else
+      bsa_fwd(q_tiles->flatten(2, 3), k_tiles->flatten(2, 3), v_tiles->flatten(2, 3), ind, cnt, scale, bs, o, false, true,
+              balance);
+    untile(o.view({B, NH, nq, bs, D}), out, gq);
+  }
+}
+
 }  // namespace
 
 TORCH_LIBRARY(li, m) {
@@ -808,6 +889,8 @@ TORCH_LIBRARY(li, m) {
   m.def("block_mask(Tensor q_pool, Tensor k_pool, int metric, int budget_mode, float ratio, int min_budget, "
         "int n_recent, bool force_diag, bool force_sink, bool force_neighbors, int nh, int nw, int num_txt_blk, "
         "int kmax, Tensor? row_budget, bool return_scores, bool k_normalized=False) -> (Tensor, Tensor, Tensor)");
+  m.def("sparse_call(Tensor q, Tensor? k_txt, Tensor? v_txt, Tensor k, Tensor v, int[] geom, int[] mask, float ratio, "
+        "Tensor? row_budget, bool fp8, bool k_norm, bool balance, Tensor(a!) out) -> ()");
   m.def("check_block_ids(Tensor ids, int n_blocks, Tensor(a!) flag) -> ()");
   m.def("bsa_fwd(Tensor q, Tensor k, Tensor v, Tensor indices, Tensor counts, float sm_scale, int block_size, "
         "Tensor(a!) out, bool return_lse, bool split, bool balance) -> Tensor");
@@ -838,6 +921,7 @@ TORCH_LIBRARY_IMPL(li, CUDA, m) {
   m.impl("kv_prep", &kv_prep);
   m.impl("untile", &untile);
   m.impl("block_mask", &block_mask);
+  m.impl("sparse_call", &sparse_call);
   m.impl("check_block_ids", &check_block_ids);
   m.impl("bsa_fwd", &bsa_fwd);
   m.impl("bsa_fwd_gather", &bsa_fwd_gather);

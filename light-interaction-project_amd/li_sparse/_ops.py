@@ -114,6 +114,11 @@ def _block_mask_fake(q_pool, k_pool, metric, budget_mode, ratio, min_budget, n_r
     return indices, counts, scores
 
 
+@torch.library.register_fake("li::sparse_call")
+def _sparse_call_fake(q, k_txt, v_txt, k, v, geom, mask, ratio, row_budget, fp8, k_norm, balance, out):
+    return None
+
+
 @torch.library.register_fake("li::check_block_ids")
 def _check_block_ids_fake(ids, n_blocks, flag):
     return None

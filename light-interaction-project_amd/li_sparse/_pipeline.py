@@ -11,10 +11,14 @@ host-side range check (the reference's ``block_indices.max()`` sync is gone).
 import math
 from dataclasses import dataclass
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
-from . import _core
+from . import _core, _lib
+from ._ops import ops
+
+_sparse_call = ops.sparse_call.default
 
 
 @dataclass(frozen=True)
@@ -300,6 +304,70 @@ def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, eve
     _call(path, q, k_txt, v_txt, k_vis, v_vis, out, g, select, text_len, events, balance, context, sorted_lists,
           normalize_k_pool)
     return out if out.dtype == out_dtype else out.to(out_dtype)
+
+
+_CALL_PLANS = {}
+
+
+def _call_plan(mode, dev, lq, lk, text_len, D, latent_hw, tile, p, default_ratio):
+    """Arguments of ``li::sparse_call`` that depend on a call's sizes and parameters only (worked out once per
+    configuration: every layer and step repeats it), or None for the calls it does not take."""
+    rb = p.get("row_budget")
+    if not (rb is None or isinstance(rb, (list, tuple, np.ndarray))):
+        return None
+    key = (mode, dev, lq, lk, text_len, D, latent_hw, tile, p.get("topk_ratio"), p.get("sim_metric"),
+           p.get("recent_protect"), p.get("force_diag"), p.get("force_sink"), p.get("qk_fp8"), default_ratio,
+           None if rb is None else tuple(rb))
+    plan = _CALL_PLANS.get(key, False)
+    if plan is not False:
+        return plan
+    g = geometry(latent_hw, tile, lq, lk, text_len)
+    fp8, plan = qk_fp8(p), None
+    if not fp8 or fp8_supported(D, tile):
+        ex = extras(p)
+        n_recent = recent_blocks(p, g.tt, g.nh, g.nw, g.nk_blk) if mode == "decode" else 0
+        budget = _lib.LI_BUDGET_HISTORY if mode == "decode" else _lib.LI_BUDGET_TOTAL
+        ratio = float(p.get("topk_ratio", 1.0 if mode == "decode" else default_ratio))
+        metric = _core.METRICS.get(p.get("sim_metric", "cosine"), _lib.LI_METRIC_DOT)
+        neighbors = mode != "decode"
+        kmax, rb_dev = _core._mask_plan(dev, g.nq_blk, g.nk_blk, g.nh, g.nw, g.num_txt_blk, n_recent, ex["force_diag"],
+                                        ex["force_sink"], neighbors, budget, ratio, 7, rb)
+        mask = [metric, budget, 7, n_recent, ex["force_diag"], ex["force_sink"], neighbors, kmax]
+        plan = ([g.H, g.W, g.tt, g.th, g.tw], [int(x) for x in mask], ratio, rb_dev, fp8, cosine(p), ragged(p))
+    if len(_CALL_PLANS) >= 64:
+        _CALL_PLANS.clear()
+    _CALL_PLANS[key] = plan
+    return plan
+
+
+def native_call(mode, q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, p, default_ratio=None):
+    """The whole call as one operator (``li::sparse_call``: the launches of ``sparse_attention``, with the host work
+    between them in C++), or None for what it leaves to ``sparse_attention``: a context cache, element types and
+    shapes that have to be converted or refused there, parameters that cannot be looked up."""
+    dt, dev, shape = q.dtype, q.device, q.shape
+    if (dt is not torch.bfloat16 and dt is not torch.float16) or dev.type != "cuda" or p.get("context_cache") is not None:
+        return None
+    if p.get("qk_fp8") and dt is not torch.bfloat16:
+        return None
+    text_len = 0 if k_txt is None else k_txt.shape[2]
+    B, NH, lq, D = shape
+    for t in (k_vis, v_vis, k_txt, v_txt) if text_len else (k_vis, v_vis):
+        if t is None or t.dtype is not dt or t.device != dev:
+            return None
+        s = t.shape
+        if len(s) != 4 or s[0] != B or s[1] != NH or s[3] != D:
+            return None
+    if k_vis.shape[2] != v_vis.shape[2] or (text_len and v_txt.shape[2] != text_len):
+        return None
+    try:
+        plan = _call_plan(mode, dev, lq, k_vis.shape[2], text_len, D, tuple(latent_hw), tile, p, default_ratio)
+    except TypeError:  # a parameter that cannot be a key
+        return None
+    if plan is None:
+        return None
+    out = torch.empty_like(q)
+    _core._run(_sparse_call, q, k_txt if text_len else None, v_txt if text_len else None, k_vis, v_vis, *plan, out)
+    return out
 
 
 def dense_attention(q, k_txt, v_txt, k_vis, v_vis):

@@ -51,6 +51,9 @@ def run_sparse_prefill_attention(q, k_txt, v_txt, k_vis, v_vis, block_idx, laten
     if current_global_chunk < 3 or q.shape[2] % (LATENT_H * LATENT_W) != 0:
         return _pipeline.dense_attention(q, k_txt, v_txt, k_vis, v_vis)
     tile = tuple(sparse_params.get("tile_size", (4, 8, 4)))
+    out = _pipeline.native_call("prefill", q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, sparse_params)
+    if out is not None:
+        return out
 
     def select(q_pool, k_pool, text_len, grid_q, grid_k, k_pool_normalized=None):
         return generate_prefill_indices(q_pool, k_pool, text_len, grid_k, dict(sparse_params, tile_size=tile),

@@ -38,13 +38,18 @@ def run_sparse_attention(q, k, v, text_len, block_idx, latent_hw, sparse_params)
         events["start"] = e
     k_txt = k[:, :, :text_len] if text_len > 0 else None
     v_txt = v[:, :, :text_len] if text_len > 0 else None
+    k_vis, v_vis = (k[:, :, text_len:], v[:, :, text_len:]) if text_len > 0 else (k, v)
+    if events is None:
+        out = _pipeline.native_call("prefill", q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, sparse_params, 0.25)
+        if out is not None:
+            return out
 
     def select(q_pool, k_pool, tl, grid_q, grid_k, k_pool_normalized=None):
         return generate_prefill_indices(q_pool, k_pool, tl, grid_k, dict(sparse_params, tile_size=tile), q.device,
                                         k_pool_normalized=k_pool_normalized)
 
     # The block mask lists every row's text blocks first (ascending ids).
-    o = _pipeline.sparse_attention(q, k_txt, v_txt, k[:, :, text_len:], v[:, :, text_len:], latent_hw, tile,
+    o = _pipeline.sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile,
                                    select, events, sorted_lists=True, balance=_pipeline.ragged(sparse_params),
                                    qk_fp8=_pipeline.qk_fp8(sparse_params),
                                    context=_pipeline.context_of(sparse_params, block_idx),
