@@ -1301,6 +1301,257 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// D = 64, BS = 64: one workgroup of 2 NE waves per 64-row query tile, NE key
+// blocks per step.
+//
+// A 64 x 64 x 64 block is 16 MFMAs and 4096 exponentials, far too little work
+// between barriers for four waves that share it and stage it through registers
+// (the kernel this replaces).  Here wave w takes the 32 query rows [32 qq, +32),
+// qq = w & 1, of every NE-th block of the list (e = w >> 1) with its own running
+// softmax, so a step has one barrier for NE blocks; the NE parts are merged once
+// at the end through LDS.  The pair of waves that shares a block loads it for
+// the next step straight to LDS (dma16_imm: one wave K, the other V, eight 1 KiB
+// chunks of 8 rows).  What bounds the large calls is the stream of blocks into
+// LDS (16 KiB for 1 MFLOP, 11 TB/s over the chip): computing S of the next block
+// beside the softmax of this one changed nothing.
+//  * K stage: 128-byte rows, the 16-byte granule g of row r at slot g ^ ((r >>
+//    1) & 7): the 16 rows of a 16-lane operand read fall in 16 distinct windows.
+//  * V stage: 128-byte rows, the 64-byte granule q of row r at q ^ ((r >> 1) &
+//    1): the four rows of a transposing read fall in the 4 distinct windows.
+// Kernel times (us; heads x tiles x blocks), before, with NE = 4 and NE = 2:
+//  4 x 64 x 16   13.4   9.9  10.5      8 x 100 x 30    54.7   51.3   40.2
+//  6 x 40 x 60   40.2  23.7  29.4      23 x 72 x 246    707    552    520
+//  8 x 40 x 30   29.0  26.5  21.2      28 x 322 x 136  1990   1655   1483
+// (NE = 1 was slower than NE = 2 at all of these but 8 x 100 x 30: 39.0.)
+template <typename E, bool G, int NE>
+__global__ __launch_bounds__(128 * NE, 2) void bsa_fwd_d64_kernel(BsaArgs a) {
+  constexpr int BS = 64, D = 64, DS = D / 16, NKT = BS / 32, NDT = D / 32, PST = BS / 16;
+  typedef typename E::vec8 vec8;
+  typedef __attribute__((address_space(3))) void lds_void;
+  // Per interleave: K (8 KiB), then V (8 KiB).
+  __shared__ __attribute__((aligned(16))) char st0[NE * 16384];
+  __shared__ __attribute__((aligned(16))) char st1[NE * 16384];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int e = wave >> 1, qq = wave & 1;
+  const int l32 = lane & 31, hl = lane >> 5;
+  const int tile = unit_tile(a, blockIdx.x);
+  const int bh = tile / a.nqt, m = tile % a.nqt;
+  const int b = bh / a.NH, h = bh % a.NH;
+  const int row0 = m * BS;
+
+  // Q^T fragments first (as in bsa_fwd_dma_kernel): lanes without a query row
+  // read row 0 of the head and keep zeros.
+  vec8 qf[DS];
+  {
+    const uint16_t* qrow;
+    bool ok;
+    if constexpr (G) {
+      const int32_t l = tile_token(a.g, a.g.Tq, m, 32 * qq + l32, ok);
+      qrow = a.q + b * a.g.qs[0] + h * a.g.qs[1] + (int64_t)(ok ? l : 0) * a.g.qs[2];
+    } else {
+      const int r = row0 + 32 * qq + l32;
+      ok = r < a.Lq;
+      qrow = a.q + ((int64_t)bh * a.Lq + (ok ? r : 0)) * D;
+    }
+#pragma unroll
+    for (int s = 0; s < DS; ++s) {
+      u32x4 x = *reinterpret_cast<const u32x4*>(qrow + 16 * s + 8 * hl);
+      if (!ok) x = u32x4{0u, 0u, 0u, 0u};
+      qf[s] = __builtin_bit_cast(vec8, x);
+    }
+  }
+  typedef __attribute__((address_space(4))) const int32_t const_i32;
+  const_i32* irow = (const_i32*)(a.idx + b * a.is[0] + h * a.is[1] + (int64_t)m * a.is[2]);
+  int count = a.cnt[b * a.cs[0] + h * a.cs[1] + (int64_t)m * a.cs[2]];
+  count = count < 0 ? 0 : (count > a.n_cols ? a.n_cols : count);
+  count = __builtin_amdgcn_readfirstlane(count);
+  const int steps = (count + NE - 1) / NE;
+
+  // This wave's load: K of its pair's block (qq = 0) or V (qq = 1).
+  const char* src = reinterpret_cast<const char*>((qq ? a.v : a.k) + (int64_t)bh * a.nkb * BS * D);
+  uint32_t voff[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const uint32_t kg = (lane & 7) ^ (lane >> 4) ^ (4 * p);
+    const uint32_t vg = 4 * (((lane & 7) >> 2) ^ ((lane >> 4) & 1)) + (lane & 3);
+    voff[p] = (lane >> 3) * 128 + 16 * (qq ? vg : kg);
+  }
+  // Block id of entry i of the list; out of range: nothing is added for it.
+  auto block_id = [&](int i) LI_INLINE { return i < count ? (int)irow[(int64_t)i * a.is[3]] : -1; };
+  auto valid = [&](int id) LI_INLINE { return (unsigned)id < (unsigned)a.nkb; };
+  auto load = [&](int id, char* st) LI_INLINE {
+    if (!valid(id)) return;
+    const char* s = src + (int64_t)id * (BS * D * 2);
+    const uint32_t dst = (uint32_t)(uintptr_t)(lds_void*)st + e * 16384 + qq * 8192;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      dma16_imm(s + (j & 4) * 1024, voff[j & 1], dst + (j & 4) * 1024, (j & 3) * 1024);
+  };
+
+  // Operand byte offsets within the interleave's stage.
+  int k_off[DS];
+  {
+    const int R = kperm(l32);  // (R + 32) >> 1 has the same low bits
+#pragma unroll
+    for (int s = 0; s < DS; ++s) k_off[s] = e * 16384 + R * 128 + 16 * ((2 * s + hl) ^ ((R >> 1) & 7));
+  }
+  const int t16 = lane & 15, g16 = lane >> 4;
+  int v_off[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+    v_off[dt] = e * 16384 + 8192 + (8 * hl + (t16 >> 2)) * 128 + 64 * (dt ^ (t16 >> 3)) + 32 * (g16 & 1) + 8 * (t16 & 3);
+
+  f32x16 o[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
+  float mrow = -__builtin_inff(), lrow = 0.0f;
+  const float qk_scale = a.qk_scale;
+
+  auto compute = [&](const char* st) LI_INLINE {
+    f32x16 sacc[NKT];
+#pragma unroll
+    for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sacc[kt][r] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < DS; ++s)
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt)
+        sacc[kt] = E::mfma32(__builtin_bit_cast(vec8, *reinterpret_cast<const u32x4*>(st + k_off[s] + 4096 * kt)), qf[s],
+                             sacc[kt]);
+    // The softmax of bsa_fwd_dma_kernel: exponentials against the running max
+    // as it stands, redone after raising it when a partial sum passes 2^20.
+    u32x4 ppk[PST];
+    auto exps = [&](float off) LI_INLINE {
+      float ls = 0.0f;
+#pragma unroll
+      for (int p = 0; p < PST; ++p) {
+        float pv[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[p >> 1][8 * (p & 1) + i], qk_scale, -off));
+        ls += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ppk[p][i] = cvt_pk<E>(pv[2 * i], pv[2 * i + 1]);
+      }
+      return ls;
+    };
+    float ls = exps(mrow);
+    if (__ballot(!(ls <= 1048576.0f))) {
+      float mx = sacc[0][0];
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, sacc[kt][r]);
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = __builtin_fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * qk_scale;
+      const float mnew = __builtin_fmaxf(mrow, mx);
+      const float msafe = mnew == -__builtin_inff() ? 0.0f : mnew;
+      const float alpha = __builtin_amdgcn_exp2f(mrow - msafe);
+      mrow = mnew;
+      lrow *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+      ls = exps(msafe);
+    }
+    lrow += ls;
+#pragma unroll
+    for (int p = 0; p < PST; ++p)
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        const uint16_t* pv = reinterpret_cast<const uint16_t*>(st + v_off[dt] + 16 * p * 128);
+        const u32x2 lo = lds_read_tr(pv), hi = lds_read_tr(pv + 4 * 64);
+        o[dt] = E::mfma32(__builtin_bit_cast(vec8, u32x4{lo[0], lo[1], hi[0], hi[1]}),
+                          __builtin_bit_cast(vec8, ppk[p]), o[dt]);
+      }
+  };
+
+  // Stage s % 2 holds the blocks of step s; those of step s + 1 land while it is
+  // computed.  The ids are read one step further ahead.
+  int id_c = block_id(e), id_n = block_id(NE + e);
+  load(id_c, st0);
+  wait_vm0();
+  __syncthreads();
+  auto step = [&](char* cur, char* nxt, int s) LI_INLINE {
+    const int id_x = id_c;
+    load(id_n, nxt);
+    id_c = id_n;
+    id_n = block_id(NE * (s + 2) + e);
+    if (valid(id_x)) compute(cur);
+    wait_vm0();
+    __syncthreads();
+  };
+  for (int s = 0; s < steps; s += 2) {
+    step(st0, st1, s);
+    if (s + 1 < steps) step(st1, st0, s + 1);
+  }
+
+  // Merge the four interleaves.  Each wave writes its O as 16-byte runs (element
+  // (dt, 4 i4 + j) of lane l at ((dt * 4 + i4) * 64 + l) * 4 + j) and its (m, l),
+  // then finishes a quarter of the head dimensions for its query rows.
+  {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lrow), __float_as_uint(lrow), false, false);
+    lrow = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  }
+  float* xo = reinterpret_cast<float*>(st0);
+  float* xm = reinterpret_cast<float*>(st1);
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4)
+      *reinterpret_cast<f32x4*>(xo + wave * 2048 + ((dt * 4 + i4) * 64 + lane) * 4) =
+          f32x4{o[dt][4 * i4], o[dt][4 * i4 + 1], o[dt][4 * i4 + 2], o[dt][4 * i4 + 3]};
+  xm[wave * 128 + lane] = mrow;
+  xm[wave * 128 + 64 + lane] = lrow;
+  __syncthreads();
+  float w[NE], mm = -__builtin_inff(), l = 0.0f;
+#pragma unroll
+  for (int x = 0; x < NE; ++x) {
+    w[x] = xm[(2 * x + qq) * 128 + lane];
+    mm = __builtin_fmaxf(mm, w[x]);
+  }
+  // A row without a block has mm = -inf: it gets zeros and an LSE of -inf.
+  const bool none = mm == -__builtin_inff();
+#pragma unroll
+  for (int x = 0; x < NE; ++x) {
+    w[x] = none ? 0.0f : __builtin_amdgcn_exp2f(w[x] - mm);
+    l += xm[(2 * x + qq) * 128 + 64 + lane] * w[x];
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const int rt = 32 * qq + l32, r = row0 + rt;
+  uint16_t* orow = nullptr;
+  if constexpr (G) {
+    bool ok;
+    const int32_t t = tile_token(a.g, a.g.Tq, m, rt, ok);
+    if (ok) orow = a.out + b * a.g.os[0] + h * a.g.os[1] + (int64_t)t * a.g.os[2];
+  } else if (r < a.Lq) {
+    orow = a.out + ((int64_t)bh * a.Lq + r) * D;
+  }
+  if (orow) {
+#pragma unroll
+    for (int k = 0; k < 8 / NE; ++k) {
+      const int run = 8 / NE * e + k;  // dt * 4 + i4
+      f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int x = 0; x < NE; ++x) {
+        const f32x4 p = *reinterpret_cast<const f32x4*>(xo + (2 * x + qq) * 2048 + (run * 64 + lane) * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += p[j] * w[x];
+      }
+      *reinterpret_cast<u32x2*>(orow + 32 * (run >> 2) + 8 * (run & 3) + 4 * hl) =
+          u32x2{cvt_pk<E>(v[0] * inv, v[1] * inv), cvt_pk<E>(v[2] * inv, v[3] * inv)};
+    }
+  }
+  if (a.lse && e == 0 && hl == 0 && r < a.Lq)
+    a.lse[(int64_t)bh * a.Lq + r] = none ? -__builtin_inff() : mm + __builtin_log2f(l);
+}
+
 // Combines the pieces of each split query tile: O = sum_e O_e a_e / sum_e l_e
 // a_e with a_e = 2^(m_e - max_e m_e); lse = max + log2(sum).  Bound by the
 // latency of the partials' loads (65 KiB a piece), so they are taken NB pieces
@@ -1375,6 +1626,21 @@ __global__ __launch_bounds__(256) void bsa_merge_kernel(BsaArgs a) {
   if (a.lse && dq == 0) a.lse[(int64_t)bh * a.Lq + r] = mm == -__builtin_inff() ? mm : mm + __builtin_log2f(l);
 }
 
+// Compute units of the current device, cached per device.
+int device_cus() {
+  static std::mutex mu;
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  std::lock_guard<std::mutex> lock(mu);
+  if (cached[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
+    cached[dev] = n > 0 ? n : -1;
+  }
+  return cached[dev] > 0 ? cached[dev] : 0;
+}
+
 // Workgroups of an attention launch: the tiles, or per XCD its whole tiles and
 // the pieces of at most xsplit split ones.
 int attn_units(const BsaArgs& a) { return a.xparts == 0 ? a.ntiles : 8 * (a.xwhole + a.xsplit * a.xparts); }
@@ -1435,27 +1701,25 @@ int launch_bsa(BsaArgs& a, hipStream_t s) {
 }
 
 template <typename E, bool QO>
+int launch_bsa_d64(BsaArgs& a, hipStream_t s) {
+  clear_launch_error();
+  // With a tile per CU at most, eight waves and four interleaves per tile; with
+  // more, four waves and two, so that two workgroups share a CU and one's loads
+  // and barriers hide behind the other's work.
+  if (a.ntiles <= device_cus())
+    hipLaunchKernelGGL((bsa_fwd_d64_kernel<E, QO, 4>), dim3(a.ntiles), dim3(512), 0, s, a);
+  else
+    hipLaunchKernelGGL((bsa_fwd_d64_kernel<E, QO, 2>), dim3(a.ntiles), dim3(256), 0, s, a);
+  return launch_status();
+}
+
+template <typename E, bool QO>
 int dispatch_bsa(BsaArgs& a, int bs, int D, hipStream_t s) {
   if (bs == 128 && D == 128) return launch_bsa_dma<E, 128, QO>(a, s);
   if (bs == 128 && D == 64) return launch_bsa<E, 128, 64, QO>(a, s);
   if (bs == 64 && D == 128) return launch_bsa_dma<E, 64, QO>(a, s);
-  if (bs == 64 && D == 64) return launch_bsa<E, 64, 64, QO>(a, s);
+  if (bs == 64 && D == 64) return launch_bsa_d64<E, QO>(a, s);
   return LI_ERR_UNSUPPORTED;
-}
-
-// Compute units of the current device, cached per device.
-int device_cus() {
-  static std::mutex mu;
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  std::lock_guard<std::mutex> lock(mu);
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
-    cached[dev] = n > 0 ? n : -1;
-  }
-  return cached[dev] > 0 ? cached[dev] : 0;
 }
 
 // Dispatch order for rows of unequal length: within each range of positions

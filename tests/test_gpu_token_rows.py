@@ -97,3 +97,38 @@ def test_rejects_what_the_kernel_does_not_take(dev):
                dict(q=torch.stack([q, q], -1)[..., 0])):
         with pytest.raises(RuntimeError):
             call(**kw)
+
+
+@pytest.mark.parametrize("H,nq", [(2, 3), (8, 40)])   # one tile per CU at most (four interleaves), more (two)
+@pytest.mark.parametrize("cols", [1, 4, 5, 11])
+def test_64_dim_kernel_against_float64(dev, H, nq, cols):
+    """Lists around the interleaves' counts, empty lists, ids out of range, a partial last tile: 2e-2 as elsewhere (P and
+    the output in bf16), LSE 1e-3."""
+    import numpy as np
+    from helpers import bits
+    from oracle import attention as oatt
+    from oracle.bf16 import bf16_to_f32
+
+    print(f"[gpu] 64-dim kernel H={H} nq={nq} cols={cols}", flush=True)
+    bs, D, nkb = 64, 64, 13
+    Lq = nq * bs - 23
+    gen = torch.Generator().manual_seed(cols)
+    q, k, v = (torch.randn(1, H, n, D, generator=gen).to(torch.bfloat16) for n in (Lq, nkb * bs, nkb * bs))
+    rng = np.random.default_rng(cols)
+    ind = np.argsort(rng.random((1, H, nq, nkb)), axis=-1)[..., :cols].astype(np.int32)
+    cnt = rng.integers(0, cols + 1, size=(1, H, nq)).astype(np.int32)
+    bad = ind.copy()
+    bad[0, 0, :, 0] = [nkb, -1, 2 ** 30][cols % 3]   # the kernel adds nothing for these
+    o, lse = _core.bsa_forward(q.to(dev), k.to(dev), v.to(dev), torch.from_numpy(bad).to(dev),
+                               torch.from_numpy(cnt).to(dev), 0.125, bs, return_lse=True)
+    torch.cuda.synchronize()
+    good, n = ind.copy(), cnt.copy()
+    for m in range(nq):
+        if n[0, 0, m] > 0:
+            good[0, 0, m, :-1], n[0, 0, m] = ind[0, 0, m, 1:], n[0, 0, m] - 1
+    f64 = lambda t: bf16_to_f32(bits(t)).astype(np.float64)  # noqa: E731
+    o_ref, lse_ref = oatt.bsa_forward(f64(q), f64(k), f64(v), good, n, 0.125, bs)
+    got, fin = lse.cpu().numpy(), np.isfinite(lse_ref)
+    assert np.array_equal(np.isneginf(got), ~fin)
+    assert np.abs(o.float().cpu().numpy() - o_ref).max() <= 2e-2
+    assert not fin.any() or np.abs(got[fin] - lse_ref[fin]).max() <= 1e-3
