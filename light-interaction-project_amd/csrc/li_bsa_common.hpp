@@ -162,20 +162,7 @@ struct Stage {
   static constexpr int value = N;
 };
 
-// 16 bytes per lane from global memory (wave-uniform base in SGPRs plus a
-// per-lane byte offset) straight into LDS at lds_addr + 16 * lane
-// (global_load_lds_dwordx4).  Issued as inline assembly so that the
-// compiler's wait-count bookkeeping does not see it: the compiler would
-// otherwise treat every pending LDS DMA as making the LDS counter unordered
-// and drain all operand reads in flight (lgkmcnt(0)) after each one.  Being
-// invisible only makes the compiler's own waits stricter (the extra loads
-// are counted by the hardware), never weaker; the caller publishes the data
-// with wait_vm0() before a barrier.  The s_nop covers the M0-write to LDS-DMA
-// hazard.
-__device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds_addr) : "memory");
-}
-// The same load with an instruction offset imm (it must fold to a constant in
+// dma16 with an instruction offset imm (it must fold to a constant in
 // [0, 4096)), which the hardware adds to both the global address
 // (sbase + voff + imm) and the LDS address (m0 + imm + 16 * lane).
 __device__ __forceinline__ void dma16_imm(const void* sbase, uint32_t voff, uint32_t m0_addr, int imm) {
@@ -215,8 +202,6 @@ __device__ __forceinline__ DmaSrc dma_sel_base(uint32_t mask, int bit, const voi
   r.voff = voff;
   return r;
 }
-__device__ __forceinline__ void wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // udiv16 with its identity mask (~0 for magic 0, else 0) passed in.
 __device__ __forceinline__ uint32_t udiv16m(uint32_t x, uint32_t magic, uint32_t id) {
   return __umulhi(x, magic) | (x & id);

@@ -48,6 +48,21 @@ struct F16 {
 
 __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) { return uint32_t(lo) | (uint32_t(hi) << 16); }
 
+// 16 bytes per lane from global memory (wave-uniform base in SGPRs plus a
+// per-lane byte offset) straight into LDS at lds_addr + 16 * lane
+// (global_load_lds_dwordx4).  Issued as inline assembly so that the
+// compiler's wait-count bookkeeping does not see it: the compiler would
+// otherwise treat every pending LDS DMA as making the LDS counter unordered
+// and drain all operand reads in flight (lgkmcnt(0)) after each one.  Being
+// invisible only makes the compiler's own waits stricter (the extra loads
+// are counted by the hardware), never weaker; the caller publishes the data
+// with wait_vm0() before a barrier.  The s_nop covers the M0-write to LDS-DMA
+// hazard.
+__device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds_addr) : "memory");
+}
+__device__ __forceinline__ void wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // x / d for x, d < 2^16 without a division: magic = ceil(2^32 / d), and 0
 // encodes d = 1.  With magic = (2^32 + e) / d, 0 <= e < d, the quotient
 // x * magic / 2^32 = x / d + x e / (d 2^32) exceeds x / d by less than 1 / d,

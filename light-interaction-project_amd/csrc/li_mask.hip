@@ -29,8 +29,8 @@
 // One wave selects each query row: every per-row reduction is a ballot +
 // popcount inside that wave, and the row's 32-bit keys live in LDS (4 bytes
 // per key block).  Aligned pools with a unit d stride take the shared-pool
-// kernel (4 rows of one head per workgroup, two waves scoring each row, the
-// head's pool streamed once through LDS tiles); other pools and very long key
+// kernel (4 rows of one head per workgroup, each wave scoring every fourth or
+// eighth chunk of 64 blocks against all of them); other pools and very long key
 // grids take the generic kernel, in which each wave scores its row by reading
 // the pool rows itself.
 #include "li_common.hpp"
@@ -49,7 +49,8 @@ struct MaskArgs {
   int32_t* indices;
   int32_t* counts;
   uint16_t* scores;
-  int32_t NH;
+  int32_t NH, NBH, groups;  // heads, batch * heads, row groups of a head (shared-pool path)
+  uint32_t mg_hw, mg_nw;  // udiv16 magics of nh nw and nw (0 for 1 and past 2^16, where no block lies)
 };
 
 __device__ __forceinline__ uint32_t order16(uint16_t bits) {
@@ -144,6 +145,21 @@ __device__ __forceinline__ void select_row(const MaskArgs& a, KeyAt&& key_at, in
     auto below = [&](int b) LI_SEL_INLINE { return b - 1 >= 16 || b - 1 < L ? b - 1 : L - 1; };
     uint32_t prefix = 0xFFFFu & ~((1u << L) - 1u);
     int b1 = 31;
+    if constexpr (KUNROLL > 4) {
+      // Many keys per lane: the counts cost more than the steps' latency, and
+      // one candidate per bit counts a third less than three per two bits.
+      for (; b1 >= 0; b1 = below(b1)) {
+        const uint32_t c = prefix | (1u << b1);
+        int n = 0;
+#pragma unroll KUNROLL
+        for (int r = 0; r < nchunk; ++r) n += wave_count(key_at(r) >= c);
+        if (n >= kk) {
+          prefix = c;
+          if (n == kk) break;
+        }
+      }
+      b1 = -1;
+    }
     while (b1 >= 0) {
       const int b0 = below(b1);
       const uint32_t m1 = 1u << b1, m0 = b0 >= 0 ? 1u << b0 : 0u;
@@ -228,29 +244,33 @@ __device__ __forceinline__ void load_query(const MaskArgs& a, int b, int h, int 
 
 // A query row's position in the key grid, for the forced-block tests.
 struct RowGeom {
-  int nk, qb, pos, hw, pt, ph, pw;
-  __device__ RowGeom(const li_mask_params& p, int qb_) : nk(p.nk), qb(qb_) {
+  int nk, qb, pos, hw, sink, pt, ph, pw;
+  __device__ RowGeom(const li_mask_params& p, int qb_, uint32_t mg_hw, uint32_t mg_nw) : nk(p.nk), qb(qb_) {
     pos = p.nk - p.nq + qb;  // query block's position in the key grid
     hw = p.nh * p.nw;
-    pt = pos / hw;
-    ph = (pos % hw) / p.nw;
-    pw = pos % p.nw;
+    sink = qb < 65536 ? qb - (int)udiv16(qb, mg_hw) * hw : qb % hw;
+    // Used for positions inside the key grid only (below 2^16).
+    pt = (int)udiv16(pos, mg_hw);
+    const int pr = pos - pt * hw;
+    ph = (int)udiv16(pr, mg_nw);
+    pw = pr - ph * p.nw;
   }
 };
 
 // Step 1b/2 for one (row, block): score bits from the fp32 dot product, the
-// forced flag, and the order key (0 for a forced block).
+// forced flag, and the order key (0 for a forced block).  mg_hw, mg_nw: udiv16
+// magics of the key grid's slab and row (nk <= kMaxNk < 2^16).
 template <typename E>
 __device__ __forceinline__ uint32_t finish_key(const li_mask_params& p, const RowGeom& g, uint16_t* srow, int j,
-                                               float dot, bool& f) {
+                                               float dot, bool& f, uint32_t mg_hw, uint32_t mg_nw) {
   uint16_t s = E::from_f32(dot);
   if (p.metric == LI_METRIC_SCALED_DOT) s = E::from_f32(E::to_f32(s) * p.scale);
   if (srow) srow[j] = s;
   f = (p.n_recent > 0) && (j >= g.nk - p.n_recent);
   if (p.force_diag && j == g.pos) f = true;
-  if (p.force_sink && j == g.qb % g.hw) f = true;
+  if (p.force_sink && j == g.sink) f = true;
   if (p.force_neighbors && g.pos >= 0 && g.pos < g.nk) {
-    const int jt = j / g.hw, jh = (j % g.hw) / p.nw, jw = j % p.nw;
+    const int jt = (int)udiv16(j, mg_hw), jr = j - jt * g.hw, jh = (int)udiv16(jr, mg_nw), jw = jr - jh * p.nw;
     if (abs(jt - g.pt) + abs(jh - g.ph) + abs(jw - g.pw) <= 1) f = true;
   }
   return f ? 0u : ((order16(s) << 16) | (0xFFFFu - (uint32_t)j));
@@ -274,7 +294,7 @@ __global__ __launch_bounds__(256) void block_mask_kernel(MaskArgs a, int waves) 
   float* qv = reinterpret_cast<float*>(keys + nk);
   load_query<E, D>(a, b, h, qb, cosine, qv, lane);
 
-  const RowGeom g(p, qb);
+  const RowGeom g(p, qb, a.mg_hw, a.mg_nw);
   const bool vec = a.ks[3] == 1 && (reinterpret_cast<uintptr_t>(a.kp) & 15u) == 0 && a.ks[0] % 8 == 0 &&
                    a.ks[1] % 8 == 0 && a.ks[2] % 8 == 0;
   const uint16_t* kbase = a.kp + b * a.ks[0] + h * a.ks[1];
@@ -296,7 +316,7 @@ __global__ __launch_bounds__(256) void block_mask_kernel(MaskArgs a, int waves) 
         for (int d = 0; d < D; ++d) ps[d & 7] = ps[d & 7] + qv[d] * x[d];
       }
       const float dot = sum8(ps);
-      keys[j] = finish_key<E>(p, g, srow, j, dot, f);
+      keys[j] = finish_key<E>(p, g, srow, j, dot, f, a.mg_hw, a.mg_nw);
     }
     nf += wave_count(f);
   }
@@ -308,146 +328,145 @@ __global__ __launch_bounds__(256) void block_mask_kernel(MaskArgs a, int waves) 
   select_row<1>(a, key_at, (nk + 63) / 64, nf, qb, bh, lane);
 }
 
-// Shared-pool path (16-byte aligned pools with unit d stride): a workgroup
-// holds 4 query rows of one (b, h), two waves per row, and streams the head's
-// pool through LDS in tiles of 128 blocks, so each pool row is read from
-// memory once per 4 query rows.  Wave (row, half) scores blocks 64 half +
-// lane of every tile against its row's query vector, held in registers.
-// Rows are padded by 16 bytes in LDS so that lanes reading consecutive
-// blocks hit distinct banks.  For cosine, thread t computes the normaliser of
-// block t of the tile and the whole workgroup then divides the tile in place
-// before the dot products.  Per (row, block) the arithmetic is the generic
-// path's: the same fp32 sums over d of the same operands.  The next
-// tile's loads are in flight while the current one is scored, and the first
-// wave of each row then selects with the row's keys in registers
-// (nk <= 64 KS).
-template <typename E, int D, int KS>
-__global__ __launch_bounds__(512) void block_mask_tiled_kernel(MaskArgs a) {
-  constexpr int NT = 128;          // blocks per tile: one per lane of a row's two waves
-  constexpr int NTHR = 512;
-  constexpr int RS = 2 * D + 16;   // LDS row stride in bytes
-  constexpr int CH = D / 8;        // 16-byte chunks per pool row
-  constexpr int PF = NT * CH / NTHR;  // 16-byte chunks per thread per tile
-  static_assert(PF * NTHR == NT * CH, "tile must split evenly over the workgroup");
-  extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+// Shared-pool path (16-byte aligned pools with unit d stride): a workgroup of
+// eight waves holds 4 query rows of one (b, h).  Waves 0-3 load and normalise a
+// query row each, while waves 4-7 stage the first chunks of 64 key blocks; SW
+// waves (4-7, then for long grids 0-3 too) score a chunk each against all four
+// rows, and waves 0-3 then finish and select a row each with the row's keys in
+// registers (nk <= 64 KS).
+//
+// The kernel is a chain of latencies (one round of workgroups at most sizes), so
+// the scoring is arranged to be short: a wave stages its chunk itself, straight
+// to LDS, a lane converts its block's row once for all four query rows, and the
+// products run on the matrix cores in fp32 (v_mfma_f32_4x4x1_16b_f32: sixteen
+// 4 x 4 outer products, block by query row, for one d).  One such step adds one
+// exact product to each sum and rounds once, as the generic path's multiply-add
+// does, so partial sum i over d = i, i + 8, ... has the same bits.
+// Kernel times, us, against one tile of 128 blocks at a time for the whole
+// workgroup with two waves per row on the vector ALU (rows x blocks):
+//   896 x 168  10.3 -> 9.9    1248 x 104 (cosine) 15.3 -> 11.4   256 x 64 (D = 64) 6.3 -> 6.1
+//   2496 x 156 24.0 -> 16.6    720 x 150 (cosine) 11.7 -> 10.5   896 x 896 27.6 -> 25.6
+template <typename E, int D, int KS, int SW>
+__global__ __launch_bounds__(512) void block_mask_rows_kernel(MaskArgs a) {
+  constexpr int CH = D / 8;           // 16-byte granules per pool row
+  constexpr int RB = 2 * D;           // bytes per pool row
+  constexpr int RPI = 1024 / RB;      // rows per load instruction
+  constexpr int QP = D + 4;           // query row pitch: the four rows in distinct banks
+  typedef __attribute__((address_space(3))) void lds_void;
+  __shared__ __attribute__((aligned(16))) char stage[SW][64 * RB];
+  __shared__ __attribute__((aligned(16))) float qall[4][QP];
+  __shared__ __attribute__((aligned(16))) float dots[4][64 * KS];
   const li_mask_params& p = a.p;
-  const int nk = p.nk;
-  uint8_t* ktile = reinterpret_cast<uint8_t*>(smem);
-  float* qall = reinterpret_cast<float*>(ktile + NT * RS);
-  float* dn = qall + 4 * D;  // cosine normalisers of the tile's blocks
-  uint32_t* kall = reinterpret_cast<uint32_t*>(dn + NT);
-  int* nf2 = reinterpret_cast<int*>(kall + (size_t)4 * nk);  // forced counts of the second waves
+  const int nk = p.nk, nchunk = (nk + 63) / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int row = wave & 3, half = wave >> 2;
-  const int qb = blockIdx.x * 4 + row;
-  const bool live = qb < p.nq;  // dead waves still take part in the tile loads and barriers
-  const int bh = blockIdx.y, b = bh / a.NH, h = bh % a.NH;
+  // Workgroup ids are dealt round-robin over the 8 XCDs; a contiguous range of
+  // (head, row group) each lets the row groups of a head share one L2's copy of
+  // its pool.
+  const int n = a.groups * a.NBH, per = n >> 3, rem = n & 7, xcd = blockIdx.x & 7;
+  const int pos = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  const int bh = pos / a.groups, b = bh / a.NH, h = bh % a.NH;
+  const int qb0 = (pos - bh * a.groups) * 4;
   const bool cosine = p.metric == LI_METRIC_COSINE;
-  float* qv = qall + row * D;
-  uint32_t* keys = kall + (size_t)row * nk;
-  if (live && half == 0) load_query<E, D>(a, b, h, qb, cosine, qv, lane);
-
-  const RowGeom g(p, qb);
   const uint16_t* kbase = a.kp + b * a.ks[0] + h * a.ks[1];
-  uint16_t* srow = (a.scores && live) ? a.scores + ((int64_t)bh * p.nq + qb) * nk : nullptr;
-  // Chunk i of this thread: tile row tid / CH + i * (NTHR / CH), column tid % CH.
-  const int r0 = tid / CH, cc = tid % CH;
-  u32x4 pf[PF];
-  // The chunks of tile rows past nt repeat the last row: every load is
-  // issued unconditionally, so they all go out together, and only rows below
-  // nt are stored.  A tile is fetched only at j0 < nk, so nt >= 1.
-  auto fetch = [&](int j0) LI_MASK_INLINE {
-    const int nt = nk - j0 < NT ? nk - j0 : NT;
+  const int sw = (wave + 4) & 7;  // scoring wave number: waves 4-7 first
+  char* st = stage[sw < SW ? sw : 0];
+
+  // Stage rows of 2 D bytes, granule g of row r at slot g ^ swz(r): the 16 lanes
+  // that read granule c of 16 consecutive rows together then hit 16 distinct
+  // windows.  Rows past nk repeat the last one; their keys are dropped.
+  auto swz = [](int r) LI_MASK_INLINE { return D == 128 ? r & 15 : (r >> 1) & 7; };
+  auto stage_chunk = [&](int chunk) LI_MASK_INLINE {
+    const uint16_t* base = kbase + (int64_t)(64 * chunk) * a.ks[2];
+    const uint32_t rstride = (uint32_t)(2 * a.ks[2]);
+    const int last = nk - 1 - 64 * chunk;
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_void*)st;
+    const int r0 = lane / CH, slot = lane % CH;
 #pragma unroll
-    for (int i = 0; i < PF; ++i) {
-      const int r = r0 + i * (NTHR / CH);
-      const int rr = r < nt ? r : nt - 1;
-      pf[i] = *reinterpret_cast<const u32x4*>(kbase + (int64_t)(j0 + rr) * a.ks[2] + 8 * cc);
+    for (int n = 0; n < 64 / RPI; ++n) {
+      const int r = n * RPI + r0;
+      const uint32_t off = (uint32_t)(r < last ? r : last) * rstride + 16u * (slot ^ swz(r));
+      dma16(base, off, lds + 1024 * n);
     }
   };
-  if (nk > 0) fetch(0);  // no key blocks: nothing to read
-  __syncthreads();  // the query rows are visible to both waves of their row
-  // The query row in registers for the dot products (wave-uniform values;
-  // stale on dead waves, never used there).
-  float qr[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) qr[d] = qv[d];
-  int nf = 0;
-  for (int j0 = 0; j0 < nk; j0 += NT) {
-    const int nt = nk - j0 < NT ? nk - j0 : NT;
-    __syncthreads();  // the previous tile is consumed
-#pragma unroll
-    for (int i = 0; i < PF; ++i) {
-      const int r = r0 + i * (NTHR / CH);
-      if (r < nt) *reinterpret_cast<u32x4*>(ktile + r * RS + 16 * cc) = pf[i];
-    }
-    __syncthreads();
-    if (j0 + NT < nk) fetch(j0 + NT);
+  const bool scores = sw < SW;
+  if (wave >= 4 && sw < nchunk) stage_chunk(sw);
+  // Rows past nq repeat the last one and are not selected.
+  if (wave < 4) load_query<E, D>(a, b, h, qb0 + wave < p.nq ? qb0 + wave : p.nq - 1, cosine, qall[wave], lane);
+  if (wave < 4 && scores && sw < nchunk) stage_chunk(sw);
+  wait_vm0();
+  __syncthreads();
+
+  // Lane l of a 4x4x1 product: A = block l, B = query row l % 4; its result
+  // element r is block 4 (l / 4) + r for query row l % 4.
+  const float* qrow = qall[lane & 3];
+  for (int chunk = scores ? sw : nchunk; chunk < nchunk; chunk += SW) {
+    if (chunk != sw) wait_vm0();
     if (cosine && !p.k_normalized) {
-      if (tid < nt) {
-        uint8_t* krow = ktile + tid * RS;
-        float ss = 0.0f;
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-          const u32x4 w = *reinterpret_cast<const u32x4*>(krow + 16 * c);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const float x = E::to_f32(uint16_t((w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu));
-            ss = ss + x * x;
-          }
-        }
-        const float nrm = E::to_f32(E::from_f32(__builtin_sqrtf(ss)));
-        const float eps = E::to_f32(E::from_f32(1e-12f));
-        dn[tid] = nrm > eps ? nrm : eps;
-      }
-      __syncthreads();
-      // The divisions, spread over the whole workgroup: each thread rewrites
-      // the chunks it stored.
-#pragma unroll
-      for (int i = 0; i < PF; ++i) {
-        const int r = r0 + i * (NTHR / CH);
-        if (r < nt) {
-          u32x4* at = reinterpret_cast<u32x4*>(ktile + r * RS + 16 * cc);
-          u32x4 w = *at;
-          const float den = dn[r];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const uint32_t lo = E::from_f32(E::to_f32(uint16_t(w[e] & 0xFFFFu)) / den);
-            const uint32_t hi = E::from_f32(E::to_f32(uint16_t(w[e] >> 16)) / den);
-            w[e] = lo | (hi << 16);
-          }
-          *at = w;
-        }
-      }
-      __syncthreads();
-    }
-    if (live) {
-      // Tile rows past nt hold stale data; their sums are computed and
-      // dropped, so the LDS reads carry no branch and can be issued ahead.
-      const int jl = lane + 64 * half;
-      float ps[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+      // The raw pool's rows, normalised in place by their lanes.
+      float ss = 0.0f;
 #pragma unroll
       for (int c = 0; c < CH; ++c) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(ktile + jl * RS + 16 * c);
+        const u32x4 w = *reinterpret_cast<const u32x4*>(st + lane * RB + 16 * (c ^ swz(lane)));
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          ps[e] = ps[e] + qr[8 * c + e] * E::to_f32(uint16_t((w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu));
+        for (int i = 0; i < 8; ++i) {
+          const float x = E::to_f32(uint16_t((w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu));
+          ss = ss + x * x;
+        }
       }
-      const float dot = sum8(ps);
-      bool f = false;
-      if (jl < nt) keys[j0 + jl] = finish_key<E>(p, g, srow, j0 + jl, dot, f);
-      nf += wave_count(f);
+      const float nrm = E::to_f32(E::from_f32(__builtin_sqrtf(ss)));
+      const float eps = E::to_f32(E::from_f32(1e-12f));
+      const float den = nrm > eps ? nrm : eps;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        u32x4* at = reinterpret_cast<u32x4*>(st + lane * RB + 16 * (c ^ swz(lane)));
+        u32x4 w = *at;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t lo = E::from_f32(E::to_f32(uint16_t(w[e] & 0xFFFFu)) / den);
+          const uint32_t hi = E::from_f32(E::to_f32(uint16_t(w[e] >> 16)) / den);
+          w[e] = lo | (hi << 16);
+        }
+        *at = w;
+      }
     }
+    f32x4 ps[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ps[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const u32x4 w = *reinterpret_cast<const u32x4*>(st + lane * RB + 16 * (c ^ swz(lane)));
+      const f32x4 q0 = *reinterpret_cast<const f32x4*>(qrow + 8 * c);
+      const f32x4 q1 = *reinterpret_cast<const f32x4*>(qrow + 8 * c + 4);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float k = E::to_f32(uint16_t((w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu));
+        ps[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(k, i < 4 ? q0[i & 3] : q1[i & 3], ps[i], 0, 0, 0);
+      }
+    }
+    // Every read of the stage has completed (its values went into the products).
+    if (chunk + SW < nchunk) stage_chunk(chunk + SW);
+    f32x4 dot;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float s8[8] = {ps[0][r], ps[1][r], ps[2][r], ps[3][r], ps[4][r], ps[5][r], ps[6][r], ps[7][r]};
+      dot[r] = sum8(s8);
+    }
+    *reinterpret_cast<f32x4*>(&dots[lane & 3][64 * chunk + 4 * (lane >> 2)]) = dot;
   }
-  if (half == 1 && lane == 0) nf2[row] = nf;
-  __syncthreads();  // both halves' keys and the second halves' counts are in LDS
-  if (!live || half == 1) return;
-  nf += nf2[row];
+  __syncthreads();
+  const int qb = qb0 + wave;
+  if (wave >= 4 || qb >= p.nq) return;
+  const RowGeom g(p, qb, a.mg_hw, a.mg_nw);
+  uint16_t* srow = a.scores ? a.scores + ((int64_t)bh * p.nq + qb) * nk : nullptr;
   uint32_t kr[KS];
+  int nf = 0;
 #pragma unroll
   for (int r = 0; r < KS; ++r) {
     const int j = r * 64 + lane;
-    kr[r] = j < nk ? keys[j] : 0u;
+    bool f = false;
+    kr[r] = 0u;
+    if (j < nk) kr[r] = finish_key<E>(p, g, srow, j, dots[wave][j], f, a.mg_hw, a.mg_nw);
+    nf += wave_count(f);
   }
   select_row<KS>(a, [&](int r) LI_MASK_INLINE { return kr[r]; }, KS, nf, qb, bh, lane);
 }
@@ -481,13 +500,6 @@ __global__ __launch_bounds__(256) void check_ids_kernel(const int32_t* ids, int6
 }
 
 constexpr int kTiledMaxNk = 64 * 28;
-
-// LDS bytes of the shared-pool path, or 0 when it does not apply.
-size_t tiled_lds(int D, int nk, bool vec_k) {
-  if (!vec_k || nk > kTiledMaxNk) return 0;
-  const size_t bytes = (size_t)128 * (2 * D + 16 + 4) + (size_t)4 * D * 4 + (size_t)4 * nk * 4 + 4 * 4;
-  return bytes <= 65536 ? bytes : 0;
-}
 
 }  // namespace
 }  // namespace li
@@ -525,28 +537,36 @@ extern "C" int li_block_mask(int dtype, int32_t B, int32_t NH, int32_t D, const 
   a.NH = NH;
   const bool vec_k = k_pool_strides[3] == 1 && (reinterpret_cast<uintptr_t>(k_pool) & 15u) == 0 &&
                      k_pool_strides[0] % 8 == 0 && k_pool_strides[1] % 8 == 0 && k_pool_strides[2] % 8 == 0;
-  const size_t tiled = tiled_lds(D, p.nk, vec_k);
+  // The shared-pool kernel keeps a chunk's row offsets in 32 bits.
+  const bool shared = vec_k && p.nk > 0 && p.nk <= kTiledMaxNk && k_pool_strides[2] >= 0 &&
+                      k_pool_strides[2] < (1ll << 24);
+  const int64_t hw = (int64_t)p.nh * p.nw;
+  a.mg_hw = hw < 65536 ? magic16((int32_t)hw) : 0x10000u;  // j / hw = 0 for every block
+  a.mg_nw = p.nw < 65536 ? magic16(p.nw) : 0x10000u;
   // Generic path: per-wave LDS slice of nk keys + the query row, up to 4
   // waves (rows) per workgroup.
   const size_t per_wave = ((size_t)p.nk + D) * 4;
   int waves = (int)(65536 / per_wave);
   waves = waves < 1 ? 1 : (waves > 4 ? 4 : waves);
-  const int rows = tiled ? 4 : waves;
-  const size_t lds = tiled ? tiled : per_wave * waves;
-  dim3 grid((unsigned)((p.nq + rows - 1) / rows), (unsigned)(B * NH));
-  dim3 block((unsigned)(tiled ? 512 : 64 * waves));
+  const int rows = shared ? 4 : waves;
+  const size_t lds = shared ? 0 : per_wave * waves;
+  a.NBH = B * NH;
+  a.groups = (p.nq + rows - 1) / rows;
+  if (shared && (int64_t)a.groups * a.NBH > 0x7FFFFFFF) return LI_ERR_SHAPE;
+  dim3 grid((unsigned)a.groups, (unsigned)(B * NH));
+  if (shared) grid = dim3((unsigned)(a.groups * a.NBH));
   hipStream_t s = static_cast<hipStream_t>(stream);
   clear_launch_error();
-#define LI_MASK_LAUNCH(E_, D_)                                                                          \
-  do {                                                                                                  \
-    if (tiled && p.nk <= 256)                                                                           \
-      hipLaunchKernelGGL((block_mask_tiled_kernel<E_, D_, 4>), grid, block, lds, s, a);                 \
-    else if (tiled && p.nk <= 1024)                                                                     \
-      hipLaunchKernelGGL((block_mask_tiled_kernel<E_, D_, 16>), grid, block, lds, s, a);                \
-    else if (tiled)                                                                                     \
-      hipLaunchKernelGGL((block_mask_tiled_kernel<E_, D_, 28>), grid, block, lds, s, a);                \
-    else                                                                                                \
-      hipLaunchKernelGGL((block_mask_kernel<E_, D_>), grid, block, lds, s, a, waves);                 \
+#define LI_MASK_LAUNCH(E_, D_)                                                                           \
+  do {                                                                                                   \
+    if (shared && p.nk <= 256)                                                                           \
+      hipLaunchKernelGGL((block_mask_rows_kernel<E_, D_, 4, 4>), grid, dim3(512), lds, s, a);            \
+    else if (shared && p.nk <= 1024)                                                                     \
+      hipLaunchKernelGGL((block_mask_rows_kernel<E_, D_, 16, 8>), grid, dim3(512), lds, s, a);           \
+    else if (shared)                                                                                     \
+      hipLaunchKernelGGL((block_mask_rows_kernel<E_, D_, 28, 8>), grid, dim3(512), lds, s, a);           \
+    else                                                                                                 \
+      hipLaunchKernelGGL((block_mask_kernel<E_, D_>), grid, dim3((unsigned)(64 * waves)), lds, s, a, waves); \
   } while (0)
   if (dtype == LI_DTYPE_BF16 && D == 128)
     LI_MASK_LAUNCH(Bf16, 128);
