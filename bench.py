@@ -387,7 +387,7 @@ def main():
     elif D == 128 and bs in (64, 128):
         kname = "bsa_fwd_dma_kernel<bf16,128>"
     else:
-        kname = f"bsa_fwd_kernel<bf16,{bs},{D}>"
+        kname = "bsa_fwd_d64_kernel<bf16>" if bs == 64 else f"bsa_fwd_kernel<bf16,{bs},{D}>"
 
     # Bytes the call moves outside attention: the pools read Q and K once
     # (fused); the tiled sequence also writes and re-reads the tiles and untiles.
@@ -541,17 +541,17 @@ def profile_kernels(args, wl, g, qd, kd, vd, q_t, q_p, k_all, v_all, k_p, params
     if fp8:
         alg["bsa_fwd_kernel"]["bytes_min_e4m3"] = (1 * (g.nq_blk + g.nk_blk) + 2 * g.nk_blk + 2 * g.nq_blk) * bs * H * D * B
         alg["bsa_fwd_kernel"]["bytes_min_e4m3_fused"] = ((g.nq_blk + g.nk_blk) * bs + 2 * (wl.lk + wl.lq)) * H * D * B
-        alg["gather_fp8_kernel<1> (Q)"] = {"bytes": H * D * B * (e * wl.lq + g.nq_blk * bs) + e * H * D * g.nq_blk}
-        alg["gather_fp8_kernel<1> (K)"] = {"bytes": H * D * B * (e * wl.lk + g.nk_blk * bs) + e * H * D * g.nk_blk}
-        alg["gather_fp8_kernel<2> (K e4m3, V)"] = {"bytes": H * D * B * (2 * e * wl.lk + (1 + e) * g.nk_blk * bs)
+        alg["prep_kernel job (Q, e4m3)"] = {"bytes": H * D * B * (e * wl.lq + g.nq_blk * bs) + e * H * D * g.nq_blk}
+        alg["prep_kernel job (K, e4m3)"] = {"bytes": H * D * B * (e * wl.lk + g.nk_blk * bs) + e * H * D * g.nk_blk}
+        alg["prep_kernel jobs (K e4m3, V)"] = {"bytes": H * D * B * (2 * e * wl.lk + (1 + e) * g.nk_blk * bs)
                                                    + e * H * D * g.nk_blk}
     elif fused:
         alg["bsa_fwd_kernel"]["bytes_min_fused"] = e * (2 * wl.lq + 2 * wl.lk) * H * D * B
         alg["pool (Q)"] = {"bytes": e * H * D * B * wl.lq + e * H * D * g.nq_blk, "grid_blocks": g.nq_blk}
         alg["pool (K)"] = {"bytes": e * H * D * B * wl.lk + e * H * D * g.nk_blk, "grid_blocks": g.nk_blk}
     else:
-        alg["gather_pool_kernel<1> (Q)"] = {"bytes": e * H * D * B * (wl.lq + g.nq_blk * bs) + e * H * D * g.nq_blk}
-        alg["gather_pool_kernel<2> (K,V)"] = {"bytes": e * H * D * B * 2 * (wl.lk + g.nk_blk * bs)
+        alg["prep_kernel job (Q)"] = {"bytes": e * H * D * B * (wl.lq + g.nq_blk * bs) + e * H * D * g.nq_blk}
+        alg["prep_kernel jobs (K, V)"] = {"bytes": e * H * D * B * 2 * (wl.lk + g.nk_blk * bs)
                                               + e * H * D * g.nk_blk}
         alg["untile_kernel"] = {"bytes": e * H * D * B * 2 * wl.lq}
     print(json.dumps({"profile": wl.name, "fused": fused, "e4m3": fp8, "launches_per_kernel": args.steps,

@@ -10,7 +10,9 @@
 // LSE m + log2(l) (longcat_kernel.py:146-155).  A row with no kept block
 // yields zeros and lse = -inf.
 //
-// Design (one workgroup = 2*BS/32 waves = one BS-row query tile; at BS = 128
+// Design of bsa_fwd_kernel, which runs D = 64 with 128-token tiles (the others:
+// bsa_fwd_dma_kernel, li_bsa_common.hpp, and bsa_fwd_d64_kernel; both keep
+// its operand layouts) (one workgroup = 2*BS/32 waves = one BS-row query tile; at BS = 128
 // that is 8 waves, two per SIMD, so one wave's softmax overlaps the other's
 // MFMAs):
 //  * wave w owns the 32 query rows [32*qq, +32) with qq = w >> 1 and the key

@@ -20,7 +20,9 @@ longcat_kernel.py:158-233), ``bsa_fwd_gather`` (the fused tile / attend /
 untile of run_sparse_attention, ar_sparse_operation.py:330-361),
 ``attn_dense`` (the dense fallback, ar_sparse_operation.py:316-317) and the
 e4m3 variants ``tile_prep_fp8``, ``kv_prep_fp8``, ``bsa_fwd_fp8``,
-``bsa_fwd_fp8_gather``.
+``bsa_fwd_fp8_gather``; ``bsa_fwd_qo`` (K and V as tiles, Q and O in token
+order), ``check_block_ids`` (longcat_kernel.py:202) and ``sparse_call`` (the
+whole of run_sparse_attention's sparse branch).
 """
 import os
 

@@ -1,11 +1,10 @@
 """The sparse-attention call shared by the HY and MG entry points.
 
 Steps (ar_sparse_operation.py:316-362, bi_sparse_operation_for_KV_cache.py:347-395,
-bi_sparse_operation.py:246-348): block geometry; tile buffers; text K/V
-zero-padded into the leading blocks; Q tile gather + pool; K/V tile gather +
-K pool; block selection; block-sparse attention; untile into ``empty_like(q)``.
-Every stage except the text copy is one HIP kernel of this package; the
-index lists come from the mask kernel, so the attention launch needs no
+bi_sparse_operation.py:246-348): block geometry; one launch that pools Q and K,
+zero-pads text K/V into the leading blocks and, where the attention kernel
+cannot read the tokens in place, gathers tiles; block selection; block-sparse
+attention into ``empty_like(q)``.  The index lists come from the mask kernel, so the attention launch needs no
 host-side range check (the reference's ``block_indices.max()`` sync is gone).
 """
 import math
