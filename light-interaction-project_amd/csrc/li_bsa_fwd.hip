@@ -673,13 +673,14 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   // element type into ppk (one u32x4 per 16-key MFMA step).
   //
   // The exponentials are taken against the running max mrow as it stands.
-  // Only when a lane's partial row sum exceeds 2^20 (some score above mrow + 20
-  // in log2 units; this includes the first block, where mrow = -inf, and
-  // non-finite scores) does the wave take the slow path: block max across
-  // both half-waves, raise mrow, rescale O and l, redo the exponentials.  So
-  // probabilities stay below 2^20 (O, l and the bf16 P far from overflow) and
-  // the block max is not computed at all on the common path; the result is
-  // the same softmax.
+  // Only when a lane's partial row sum exceeds E::kMaxPartSum (2^20 in bf16,
+  // 2^15 in half precision: some score about as many log2 units above mrow;
+  // this includes the first block, where mrow = -inf, and non-finite scores)
+  // does the wave take the slow path: block max across both half-waves, raise
+  // mrow, rescale O and l, redo the exponentials.  So no probability exceeds
+  // that bound, which keeps O and l far from overflow in fp32 and P finite in
+  // the element type it is rounded to, and the block max is not computed at
+  // all on the common path; the result is the same softmax.
   u32x4 ppk[C::PST];
   auto exps = [&](float off) LI_INLINE {
     float ls = 0.0f;
@@ -702,7 +703,7 @@ __global__ __launch_bounds__(4 * BS) void bsa_fwd_dma_kernel(BsaArgs a) {
   // exponentials against 0 instead (all zero), never against -inf.
   auto softmax = [&]() LI_INLINE {
     float ls = exps(mrow);
-    if (__ballot(!(ls <= 1048576.0f))) {
+    if (__ballot(!(ls <= E::kMaxPartSum))) {
       float mx = sacc[0][0];
 #pragma unroll
       for (int kt = 0; kt < C::NKT; ++kt)
@@ -1426,7 +1427,8 @@ __global__ __launch_bounds__(128 * NE, 2) void bsa_fwd_d64_kernel(BsaArgs a) {
         sacc[kt] = E::mfma32(__builtin_bit_cast(vec8, *reinterpret_cast<const u32x4*>(st + k_off[s] + 4096 * kt)), qf[s],
                              sacc[kt]);
     // The softmax of bsa_fwd_dma_kernel: exponentials against the running max
-    // as it stands, redone after raising it when a partial sum passes 2^20.
+    // as it stands, redone after raising it when a partial sum passes
+    // E::kMaxPartSum, so that P stays finite in the element type.
     u32x4 ppk[PST];
     auto exps = [&](float off) LI_INLINE {
       float ls = 0.0f;
@@ -1443,7 +1445,7 @@ __global__ __launch_bounds__(128 * NE, 2) void bsa_fwd_d64_kernel(BsaArgs a) {
       return ls;
     };
     float ls = exps(mrow);
-    if (__ballot(!(ls <= 1048576.0f))) {
+    if (__ballot(!(ls <= E::kMaxPartSum))) {
       float mx = sacc[0][0];
 #pragma unroll
       for (int kt = 0; kt < NKT; ++kt)

@@ -16,9 +16,14 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // Element-type traits: storage is always 16-bit; conversion to/from fp32 and
-// the matching 32x32x16 MFMA differ.
+// the matching 32x32x16 MFMA differ.  kMaxPartSum: the largest partial sum of
+// probabilities of a lane that the attention kernels let pass before they raise
+// their running max.  It bounds every probability, which is rounded to the
+// element type: bf16 has fp32's range, a half ends at 65504 (above 65520 it
+// rounds to infinity), hence 2^15.
 struct Bf16 {
   typedef bf16x8 vec8;
+  static constexpr float kMaxPartSum = 1048576.0f;  // 2^20
   static __device__ __forceinline__ float to_f32(uint16_t b) { return __uint_as_float(uint32_t(b) << 16); }
   static __device__ __forceinline__ uint16_t from_f32(float x) {
     __bf16 h = (__bf16)x;  // round to nearest even
@@ -31,6 +36,7 @@ struct Bf16 {
 
 struct F16 {
   typedef f16x8 vec8;
+  static constexpr float kMaxPartSum = 32768.0f;  // 2^15
   static __device__ __forceinline__ float to_f32(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
   // The empty asm keeps x an fp32 value: otherwise the compiler may fold the
   // multiply-add that produced x into the conversion (v_fma_mixlo_f16), one
