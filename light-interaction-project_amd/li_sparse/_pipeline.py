@@ -9,6 +9,8 @@ host-side range check (the reference's ``block_indices.max()`` sync is gone).
 """
 import math
 from dataclasses import dataclass
+from numbers import Real
+from operator import index
 
 import numpy as np
 import torch
@@ -310,29 +312,39 @@ _CALL_PLANS = {}
 
 def _call_plan(mode, dev, lq, lk, text_len, D, latent_hw, tile, p, default_ratio):
     """Arguments of ``li::sparse_call`` that depend on a call's sizes and parameters only (worked out once per
-    configuration: every layer and step repeats it), or None for the calls it does not take."""
-    rb = p.get("row_budget")
-    if not (rb is None or isinstance(rb, (list, tuple, np.ndarray))):
+    configuration: every layer and step repeats it), or None for the calls it does not take.
+
+    A configuration is looked up by the values that its parameters resolve to, read anew for each call: an absent key
+    and an explicit None are not the same for all of them, and a parameter may be an object that changes in place.
+    """
+    (H, W), (tt, th, tw) = latent_hw, tile
+    latent_hw, tile = (index(H), index(W)), (index(tt), index(th), index(tw))
+    fp8, decode = qk_fp8(p), mode == "decode"
+    if fp8 and not fp8_supported(D, tile):
         return None
-    key = (mode, dev, lq, lk, text_len, D, latent_hw, tile, p.get("topk_ratio"), p.get("sim_metric"),
-           p.get("recent_protect"), p.get("force_diag"), p.get("force_sink"), p.get("qk_fp8"), default_ratio,
-           None if rb is None else tuple(rb))
-    plan = _CALL_PLANS.get(key, False)
-    if plan is not False:
+    rb, rb_key = p.get("row_budget"), None
+    if rb is not None:
+        rb = np.asarray(rb) if isinstance(rb, (list, tuple, np.ndarray)) else None
+        if rb is None or rb.ndim != 1 or rb.dtype.kind not in "iub":
+            return None
+        rb_key = (rb.dtype.str, rb.tobytes())
+    protect = p.get("recent_protect", 0) if decode else 0
+    if not isinstance(protect, Real):
+        return None
+    diag, sink = bool(p.get("force_diag", False)), bool(p.get("force_sink", False))
+    ratio = float(p.get("topk_ratio", 1.0 if decode else default_ratio))
+    metric, cos = _core.METRICS.get(p.get("sim_metric", "cosine"), _lib.LI_METRIC_DOT), cosine(p)
+    key = (decode, dev, lq, lk, text_len, D, latent_hw, tile, ratio, metric, cos, protect, diag, sink, fp8, rb_key)
+    plan = _CALL_PLANS.get(key)
+    if plan is not None:
         return plan
     g = geometry(latent_hw, tile, lq, lk, text_len)
-    fp8, plan = qk_fp8(p), None
-    if not fp8 or fp8_supported(D, tile):
-        ex = extras(p)
-        n_recent = recent_blocks(p, g.tt, g.nh, g.nw, g.nk_blk) if mode == "decode" else 0
-        budget = _lib.LI_BUDGET_HISTORY if mode == "decode" else _lib.LI_BUDGET_TOTAL
-        ratio = float(p.get("topk_ratio", 1.0 if mode == "decode" else default_ratio))
-        metric = _core.METRICS.get(p.get("sim_metric", "cosine"), _lib.LI_METRIC_DOT)
-        neighbors = mode != "decode"
-        kmax, rb_dev = _core._mask_plan(dev, g.nq_blk, g.nk_blk, g.nh, g.nw, g.num_txt_blk, n_recent, ex["force_diag"],
-                                        ex["force_sink"], neighbors, budget, ratio, 7, rb)
-        mask = [metric, budget, 7, n_recent, ex["force_diag"], ex["force_sink"], neighbors, kmax]
-        plan = ([g.H, g.W, g.tt, g.th, g.tw], [int(x) for x in mask], ratio, rb_dev, fp8, cosine(p), ragged(p))
+    n_recent = recent_blocks(p, g.tt, g.nh, g.nw, g.nk_blk) if decode else 0
+    budget = _lib.LI_BUDGET_HISTORY if decode else _lib.LI_BUDGET_TOTAL
+    kmax, rb_dev = _core._mask_plan(dev, g.nq_blk, g.nk_blk, g.nh, g.nw, g.num_txt_blk, n_recent, diag, sink, not decode,
+                                    budget, ratio, 7, rb)
+    mask = [metric, budget, 7, n_recent, diag, sink, not decode, kmax]
+    plan = ([g.H, g.W, g.tt, g.th, g.tw], [int(x) for x in mask], ratio, rb_dev, fp8, cos, rb is not None)
     if len(_CALL_PLANS) >= 64:
         _CALL_PLANS.clear()
     _CALL_PLANS[key] = plan
@@ -359,8 +371,8 @@ def native_call(mode, q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, p, default
     if k_vis.shape[2] != v_vis.shape[2] or (text_len and v_txt.shape[2] != text_len):
         return None
     try:
-        plan = _call_plan(mode, dev, lq, k_vis.shape[2], text_len, D, tuple(latent_hw), tile, p, default_ratio)
-    except TypeError:  # a parameter that cannot be a key
+        plan = _call_plan(mode, dev, lq, k_vis.shape[2], text_len, D, latent_hw, tile, p, default_ratio)
+    except TypeError:  # a parameter that the general route refuses or converts
         return None
     if plan is None:
         return None
