@@ -1596,15 +1596,18 @@ __global__ __launch_bounds__(256) void bsa_merge_kernel(BsaArgs a) {
     float mx = mm;
 #pragma unroll
     for (int i = 0; i < NB; ++i) mx = __builtin_fmaxf(mx, ml[i][0]);
-    if (mx == -__builtin_inff()) continue;  // nothing kept so far
-    const float keep = __builtin_amdgcn_exp2f(mm - mx);
+    // With no score above -inf so far every weight is 0, taken against 0: the
+    // sums stay 0, or NaN for a row whose scores are all NaN (m = -inf, l and O
+    // NaN), as a whole tile gives it.
+    const float base = mx == -__builtin_inff() ? 0.0f : mx;
+    const float keep = __builtin_amdgcn_exp2f(mm - base);
     mm = mx;
     l *= keep;
 #pragma unroll
     for (int d = 0; d < 8; ++d) acc[d] *= keep;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const float w = e0 + i < a.xparts ? __builtin_amdgcn_exp2f(ml[i][0] - mx) : 0.0f;
+      const float w = e0 + i < a.xparts ? __builtin_amdgcn_exp2f(ml[i][0] - base) : 0.0f;
       l += ml[i][1] * w;
 #pragma unroll
       for (int d = 0; d < 8; ++d) acc[d] += o[i][d >> 2][d & 3] * w;

@@ -100,3 +100,26 @@ def test_token_order_pieces_equal_tiled_pieces(dev):
                 for f in (True, False))
         torch.cuda.synchronize()
         assert a.dtype == dtype and torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+def test_nan_rows_stay_nan_when_split(dev):
+    """A NaN in a query row (every score NaN) or in a key gives NaN outputs from split tiles as from whole ones."""
+    bs, D, H, nq, cols = 128, 128, 2, 4, 40
+    print(f"[gpu] NaN rows: room for {_pieces(H, nq * bs, cols, dev)} pieces", flush=True)
+    assert _pieces(H, nq * bs, cols, dev) >= 16
+    q, k, v = _bf16(1, (1, H, nq * bs, D), 0.3), _bf16(2, (1, H, cols * bs, D)), _bf16(3, (1, H, cols * bs, D))
+    q[0, 0, 5, 7] = q[0, 1, 200] = float("nan")
+    k[0, 1, 9 * bs + 3, 2] = float("nan")
+    ind = torch.arange(cols, dtype=torch.int32, device=dev).repeat(1, H, nq, 1)
+    cnt = torch.full((1, H, nq), cols, dtype=torch.int32, device=dev)
+    cnt[0, 1, 2:] = 9            # lists that end before the key with the NaN
+    scale = 1.0 / math.sqrt(D)
+    got = [_core.bsa_forward(q.to(dev), k.to(dev), v.to(dev), ind, cnt, scale, bs, return_lse=True, split=s)
+           for s in (True, False)]
+    torch.cuda.synchronize()
+    (out_s, _), (out_w, _) = got
+    want = torch.zeros(1, H, nq * bs, dtype=torch.bool, device=dev)
+    want[0, 0, 5] = want[0, 1, :2 * bs] = True
+    for out in (out_s, out_w):
+        assert torch.equal(torch.isnan(out).any(-1), want) and torch.equal(torch.isnan(out).all(-1), want)
+    assert (out_s.float() - out_w.float())[~want].abs().max().item() <= 1e-2
