@@ -1792,38 +1792,50 @@ constexpr int64_t kPartBytes = 128 * (128 + 2) * 4;  // one piece: O and (m, l) 
 // All pieces of a launch fit the scratch of the allocation-free entry point.
 constexpr int64_t kMaxPartBytes = 32ll << 20;
 
-// Time (us) of n units of `blocks` blocks each on c CUs: 9 us per unit (its
-// prologue, first softmax, epilogue and the CU's next dispatch) and 1.55 us per
-// block with every CU busy.  A block takes less when part of the chip idles,
-// down to 1.0 us at half of the CUs: the kernel runs at the card's power limit
-// (16 heads x 56 tiles x 51 blocks take 331 us on random data, 218 on zeros).
+// Price (us) of n units of `blocks` blocks each on c CUs: 9.5 us per unit (its
+// prologue, first softmax, epilogue and the CU's next dispatch) and 1.3 us per
+// block with every CU busy, down to 1.1 us at half of the CUs (the kernel runs
+// at the card's power limit, so a block takes less when part of the chip idles).
 double units_us(int64_t n, double blocks, int64_t c) {
-  constexpr double kUnit = 9.0, kBlock = 1.55, kBlockIdle = 1.0;
+  constexpr double kUnit = 9.5, kBlock = 1.3, kBlockIdle = 1.1;
   const double u = (double)(n % c) / (double)c;
   const double last = u <= 0.5 ? kBlockIdle : kBlockIdle + (kBlock - kBlockIdle) * (u - 0.5) / 0.5;
   return (double)(n / c) * (kUnit + blocks * kBlock) + (n % c ? kUnit + blocks * last : 0.0);
 }
 
 // The plan for lists of up to n_cols blocks within `bytes` of partials.  The
-// model's figures are within 10% of the measured ones at every size below
-// (attention and merge, us, bf16; heads x tiles x blocks):
-//   1 x  8 x 60: whole 67.2, 10 pieces 20.1   1 x 52 x 24: 31.6, 4 pieces 23.6
-//   1 x 52 x 72: 79.6, 4 pieces 40.0          2 x 52 x 40: 48.0, 2 pieces 41.9
-//   8 x 36 x 30: 92.8, 6 pieces 74.7          8 x 44 x 40: 118.9, 2 pieces 110.6
-//  16 x 49 x 50: 321.8, 8 pieces 284.7       16 x 56 x 51: 329.1, 2 pieces 325.2
-// and whole tiles stay the better ones at 3 x 52 x 72 (92.5 against 96.9), 2 x
-// 52 x 16 (24.0, 29.6), 1 x 52 x 8 (15.9, 18.5) and 8 x 58 x 39 (132.2, 145.4).
+// pieces pay for writing their partials (65 KiB each) and for the merge that
+// reads them: 3 us and 0.019 us per piece after earlier rounds, whose tiles end
+// at different times; 1 us and 0.046 us per piece in a launch of one round, where
+// all the pieces write at once.
+//
+// The constants were fitted to the choice, not to the times: over 225 sizes (8
+// to 1500 tiles of 8 to 80 blocks), each run whole and with 2 to 16 pieces in bf16
+// and in e4m3, the chosen number is within 0.2% of the best one in the mean (7% at
+// worst), and at most 1% (one e4m3 size 3%) slower than two pieces behind a last
+// round at most half full and whole tiles otherwise.  One merge price for both
+// kinds of launch lost 1 to 9% to that at lists of 12 to 36 blocks behind a last
+// round about half full, and 5% with pieces of short lists in a small launch.
+// Attention and merge, us (tiles x blocks; f16 as bf16):
+//     8 x 60  bf16:  66.6, 10 pieces 20.1       52 x 16  bf16: 23.9, 2 pieces 22.6, 4 pieces 23.4
+//   104 x 40  bf16:  51.2,  2 pieces 41.8       52 x 16  e4m3: 21.9, 2 pieces 20.7, 4 pieces 23.1
+//   352 x 24  bf16:  81.9,  2 pieces 76.4      352 x 24  e4m3: 70.9, 2 pieces 65.3
+//   384 x 36  bf16: 117.1,  2 pieces 110.3     384 x 36  e4m3: 101.7, 2 pieces 92.9
+//   784 x 50  bf16: 320.9, 10 pieces 285.7     896 x 36  e4m3: 207.7, 2 pieces 198.9
+//   896 x 51  bf16: 329.6,  2 pieces 324.4     896 x 36  bf16: 245.5, 2 pieces 238.6
+// and whole tiles stay the better ones at 104 x 16 (25.5 against 29.7), 52 x 8 (16.3,
+// 18.7), 160 x 40 (59.6, 66.2) and 472 x 36 (125.5, 140.8).
 SplitPlan plan_split(int64_t tiles, int64_t n_cols, int cus, int64_t bytes) {
-  constexpr double kMerge = 5.5, kMergePiece = 0.012;  // the merge launch, and its read of one piece
   SplitPlan best;
   if (cus <= 0 || cus % 8 != 0 || n_cols <= 0) return best;
   const int64_t n = (tiles + 7) / 8, c = cus / 8, r = n % c;
   if (r == 0) return best;
+  const double merge = n < c ? 1.0 : 3.0, merge_piece = n < c ? 0.046 : 0.019;
   const int64_t most = (bytes < kMaxPartBytes ? bytes : kMaxPartBytes) / (8 * kPartBytes);  // pieces per XCD
   double cost = units_us(r, (double)n_cols, c) - 1.0;  // a gain of less than 1 us is left
   for (int64_t parts = 2; parts * r <= most && parts <= n_cols; ++parts) {
     const double blocks = (double)((n_cols + parts - 1) / parts);
-    const double t = units_us(r * parts, blocks, c) + kMerge + kMergePiece * 8.0 * (double)(r * parts);
+    const double t = units_us(r * parts, blocks, c) + merge + merge_piece * 8.0 * (double)(r * parts);
     if (t < cost) {
       cost = t;
       best.whole = (int32_t)(n - r);

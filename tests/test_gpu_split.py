@@ -63,6 +63,17 @@ def test_pieces_match_whole_tiles_and_oracle(dev, H, nq, cols):
         assert np.abs(got[b, h, rows] - o_ref[b, h, rows]).max() <= 2e-2
 
 
+@pytest.mark.parametrize("H,nq,cols,parts", [(16, 22, 24, 2), (16, 24, 36, 2), (16, 56, 36, 2), (16, 56, 51, 2),
+                                             (2, 26, 16, 2), (2, 52, 16, 0), (2, 26, 8, 0), (16, 28, 36, 0)])
+def test_pieces_of_the_faster_choice(dev, H, nq, cols, parts):
+    """Lists of 12 to 36 blocks behind a last round at most half full run as two pieces (the first three were whole, 3-9%
+    slower), a small launch with short lists as two (not four: 3-8% slower) or whole, as do fuller last rounds."""
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the sizes are those of 256 CUs")
+    n = -(-H * nq // 8)
+    assert _pieces(H, nq * 128, cols, dev) == 8 * (n % 32) * parts
+
+
 @pytest.mark.parametrize("H,Lq,Lk,txt", [(1, 300, 1500, 0), (2, 640, 2052, 300), (16, 6240, 3072, 77)])
 def test_dense_pieces_match_whole_tiles(dev, H, Lq, Lk, txt):
     q, k, v = (_bf16(s, (1, H, n, 128)).to(dev) for s, n in ((4, Lq), (5, Lk), (6, Lk)))
