@@ -4,8 +4,8 @@ Steps (ar_sparse_operation.py:316-362, bi_sparse_operation_for_KV_cache.py:347-3
 bi_sparse_operation.py:246-348): block geometry; one launch that pools Q and K,
 zero-pads text K/V into the leading blocks and, where the attention kernel
 cannot read the tokens in place, gathers tiles; block selection; block-sparse
-attention into ``empty_like(q)``.  The index lists come from the mask kernel, so the attention launch needs no
-host-side range check (the reference's ``block_indices.max()`` sync is gone).
+attention into ``empty_like(q)``.  The index lists come from the mask kernel, so
+the attention launch needs no host-side range check (the reference's ``block_indices.max()`` sync is gone).
 """
 import math
 from dataclasses import dataclass
@@ -145,23 +145,19 @@ def _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm):
 
     path: "fused" (pools; padded text K/V), "fused_fp8" (e4m3 Q and K tiles + scales, pools; padded text V), "mixed"
     (K, V tiles, pools), "tiled" (Q, K, V tiles, pools), "mixed_fp8" and "tiled_fp8" (e4m3 Q and K tiles + scales, V
-    tiles, pools).  Query-side buffers are the call's own; key-side ones (text blocks, then the visual blocks from the first uncached frame) are the
-    ContextCache's where there is one.  k_norm: also keep the K pool's rows normalised for the cosine selection
-    (``k_pool_n``; the selection takes it as ``k_pool_normalized``).
+    tiles, pools).  Query-side buffers are the call's own; key-side ones (text blocks, then the visual blocks from the
+    first uncached frame) are the ContextCache's where there is one.  k_norm: also keep the K pool's rows normalised for
+    the cosine selection (``k_pool_n``; the selection takes it as ``k_pool_normalized``).
     """
     B, NH, _, D = q.shape
     dt = q.dtype
     fp8, tiled = path.endswith("_fp8"), not path.startswith("fused")
-    if path == "fused" and text_len > 0:
-        _core._same_dtype(q, k_txt, v_txt)
-    elif text_len > 0:
-        k_txt, v_txt = k_txt.to(dt), v_txt.to(dt)
     cache, layer, cframes = ctx if ctx is not None else (None, None, 0)
     cf = min((max(cframes, 0) // g.tt) * g.tt, g.T_k) if cache is not None else 0
     key = (path, layer, B, NH, D, dt, str(q.device), g, text_len, cf, bool(k_norm)) if cache is not None else None
     bufs = cache._entries.get(key) if cache is not None else None
     first = cf if bufs is not None else 0
-    text, padded = None, (None, None)
+    text, padded, k_codes = None, (None, None), None
     if bufs is None:
         nkb = g.num_txt_blk + g.nk_blk
         bufs = dict.fromkeys(("k_pool_n", "k8", "k_scale", "k_all", "v_all", "kt", "vt"))
@@ -176,6 +172,16 @@ def _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm):
         if tiled:
             bufs["v_all"] = q.new_empty((B, NH, nkb, g.bs, D))
         if text_len > 0:
+            if tiled:
+                # Tiles take text of another element type (16-bit ones of another device too) as a copy into them
+                # would; e4m3 codes are those of the 16-bit keys as they came.
+                if fp8:
+                    _core._device_check(q, k_txt)
+                    _core.dtype_code(k_txt)
+                    k_codes = k_txt if k_txt.dtype != dt else None
+                k_txt, v_txt = k_txt.to(q), v_txt.to(q)
+            else:
+                _core._same_dtype(q, k_txt, v_txt)
             text = (k_txt, v_txt)
             # Whole blocks of text are read where they are.
             whole = text_len % g.bs == 0
@@ -198,6 +204,8 @@ def _prepare(path, q, k_txt, v_txt, k_vis, v_vis, g, text_len, ctx, k_norm):
                (g.T_k - first, *rest), q_tiles=out["q_tiles"], q_scale=out["q_scale"],
                k_tiles=bufs["k8"] if fp8 else bufs["k_all"], k_scale=bufs["k_scale"], v_tiles=bufs["v_all"],
                k_pool_n=bufs["k_pool_n"], num_txt_blk=g.num_txt_blk, text=text, padded_text=padded)
+    if k_codes is not None:
+        _core.tile_prep_fp8(k_codes, bufs["k8"], bufs["k_scale"], None, 0, 0, 1, 1, text_len, 1, 1, g.bs, 1, g.num_txt_blk)
     if cache is not None:
         cache._entries[key] = bufs
     return out
@@ -274,8 +282,8 @@ def sparse_attention(q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, select, eve
     shape allows it (D = 128, 128-token tiles, tw and W multiples of 4, a grid
     at least one tile high and wide, token views with unit d stride);
     otherwise, or with ``fused=False``, K and V are tiled first and the kernel reads Q and writes O in
-    token order (or Q is tiled and O untiled too, for views it cannot read).  All give the same bits.  ``balance`` (rows with their own budgets) starts
-    the longest query tiles first.  ``qk_fp8`` takes Q K^T on e4m3 codes with one scale per tile
+    token order (or Q is tiled and O untiled too, for views it cannot read).  All give the same bits.
+    ``balance`` (rows with their own budgets) starts the longest query tiles first.  ``qk_fp8`` takes Q K^T on e4m3 codes with one scale per tile
     block (bf16 only; D = 128 and 128-token tiles, ValueError otherwise); the selection is unchanged.
     ``context`` = (ContextCache, layer key, context frames) keeps the key-side preparation of the
     fixed leading frames and the text across calls (see ContextCache).  ``normalize_k_pool`` (``select``

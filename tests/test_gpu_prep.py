@@ -116,3 +116,44 @@ def test_prep_rejects_short_tensors(dev):
                 dict(q_tiles=short), dict(k_pool_n=pool[:, :1])):
         with pytest.raises(RuntimeError):
             call(**bad)
+
+
+@pytest.mark.parametrize("text", [77, 128])
+def test_text_of_another_type_or_device(dev, text):
+    """K / V tiles take text as a copy into them would; e4m3 codes are those of the 16-bit text keys as they came;
+    what reads the text in place, or quantizes 32-bit keys, refuses it."""
+    from li_sparse import ContextCache, _pipeline
+    from li_sparse.hy.ar_sparse_operation import fast_generate_indices
+
+    print(f"[gpu] text of another type: {text} tokens", flush=True)
+    gen, tile, NH, D = torch.Generator().manual_seed(9), (4, 8, 4), 2, 128
+    params = {"tile_size": tile, "topk_ratio": 0.5, "sim_metric": "scaled_dot_product"}
+    kt, vt = (torch.randn(1, NH, text, D, generator=gen).to(dev) for _ in range(2))
+
+    def call(hw, kt, vt, fp8, cache=None):
+        q, k = (_tok(torch.Generator().manual_seed(f), 1, NH, f * hw[0] * hw[1], D, torch.bfloat16, dev, "bhld")
+                for f in (3, 5))
+        return _pipeline.sparse_attention(
+            q, kt, vt, k, k, hw, tile, lambda qp, kp, tl, gq, gk: fast_generate_indices(qp, kp, tl, gq, gk, params, dev),
+            qk_fp8=fp8, context=(cache, 0, 4) if cache is not None else None)
+
+    odd, even = (9, 13), (9, 16)       # K / V tiles; tokens read in place
+    ref = call(odd, kt.bfloat16(), vt.bfloat16(), False)
+    for a, b in ((kt, vt), (kt.cpu(), vt.cpu()), (kt.bfloat16(), vt.cpu())):
+        assert torch.equal(_bits(call(odd, a, b, False)), _bits(ref))
+    cache, n = ContextCache(), -(-text // 128)
+    half = kt.half()
+    out = call(odd, half, vt, True, cache)
+    bufs = next(iter(cache._entries.values()))
+    codes = torch.empty((1, NH, n, 128, D), dtype=torch.float8_e4m3fn, device=dev)
+    scales = torch.empty((1, NH, n), device=dev)
+    rows = torch.nn.functional.pad(half, (0, 0, 0, n * 128 - text))
+    _core.tile_prep_fp8(rows, codes, scales, None, 0, 0, n, 1, 128, 1, 1, 128, 1, 1)
+    assert torch.equal(_bits(bufs["k8"][:, :, :n].contiguous()), _bits(codes))
+    assert torch.equal(_bits(bufs["k_scale"][:, :, :n].contiguous()), _bits(scales))
+    assert torch.equal(_bits(call(odd, half, vt, True, cache)), _bits(out))   # the second call keeps them
+    for hw, a, b, fp8 in ((odd, kt, vt, True), (even, kt, vt.bfloat16(), True), (even, half, half, True),
+                          (even, kt.bfloat16(), vt, False), (even, half, half, False)):
+        with pytest.raises((TypeError, RuntimeError)):
+            call(hw, a, b, fp8)
+    torch.cuda.synchronize()
