@@ -1496,9 +1496,9 @@ __global__ __launch_bounds__(128 * NE, 2) void bsa_fwd_d64_kernel(BsaArgs a) {
     if (s + 1 < steps) step(st1, st0, s + 1);
   }
 
-  // Merge the four interleaves.  Each wave writes its O as 16-byte runs (element
+  // Merge the NE interleaves.  Each wave writes its O as 16-byte runs (element
   // (dt, 4 i4 + j) of lane l at ((dt * 4 + i4) * 64 + l) * 4 + j) and its (m, l),
-  // then finishes a quarter of the head dimensions for its query rows.
+  // then finishes 1 / NE of the head dimensions for its query rows.
   {
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lrow), __float_as_uint(lrow), false, false);
     lrow = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
@@ -1552,8 +1552,9 @@ __global__ __launch_bounds__(128 * NE, 2) void bsa_fwd_d64_kernel(BsaArgs a) {
           u32x2{cvt_pk<E>(v[0] * inv, v[1] * inv), cvt_pk<E>(v[2] * inv, v[3] * inv)};
     }
   }
+  // A row whose scores are all NaN has mm = -inf too, but a NaN sum: its LSE is NaN.
   if (a.lse && e == 0 && hl == 0 && r < a.Lq)
-    a.lse[(int64_t)bh * a.Lq + r] = none ? -__builtin_inff() : mm + __builtin_log2f(l);
+    a.lse[(int64_t)bh * a.Lq + r] = none && l == 0.0f ? -__builtin_inff() : mm + __builtin_log2f(l);
 }
 
 // Combines the pieces of each split query tile: O = sum_e O_e a_e / sum_e l_e

@@ -132,3 +132,23 @@ def test_64_dim_kernel_against_float64(dev, H, nq, cols):
     assert np.array_equal(np.isneginf(got), ~fin)
     assert np.abs(o.float().cpu().numpy() - o_ref).max() <= 2e-2
     assert not fin.any() or np.abs(got[fin] - lse_ref[fin]).max() <= 1e-3
+
+
+@pytest.mark.parametrize("H,nq", [(2, 3), (8, 40)])
+def test_64_dim_kernel_keeps_nan(dev, H, nq):
+    """A query row with a NaN (every score NaN) has NaN outputs and a NaN LSE; an empty list zeros and -inf."""
+    print(f"[gpu] 64-dim kernel, NaN rows H={H} nq={nq}", flush=True)
+    bs, D, nkb = 64, 64, 6
+    gen = torch.Generator().manual_seed(1)
+    q, k, v = (torch.randn(1, H, n * bs, D, generator=gen).to(torch.bfloat16).to(dev) for n in (nq, nkb, nkb))
+    q[0, 0, 5, 7] = q[0, 1, bs + 60] = float("nan")
+    ind = torch.arange(nkb, dtype=torch.int32, device=dev).repeat(1, H, nq, 1)
+    cnt = torch.full((1, H, nq), nkb, dtype=torch.int32, device=dev)
+    cnt[0, 0, 1] = 0
+    o, lse = _core.bsa_forward(q, k, v, ind, cnt, 0.125, bs, return_lse=True)
+    torch.cuda.synchronize()
+    want = torch.zeros(1, H, nq * bs, dtype=torch.bool, device=dev)
+    want[0, 0, 5] = want[0, 1, bs + 60] = True
+    assert torch.equal(torch.isnan(o).all(-1), want) and torch.equal(torch.isnan(o).any(-1), want)
+    assert torch.equal(torch.isnan(lse), want)
+    assert torch.isneginf(lse[0, 0, bs:2 * bs]).all() and not o[0, 0, bs:2 * bs].any()
