@@ -17,6 +17,7 @@
 //   hy-worldplay/.../longcat_kernel.py:158-233 (longcat_flash_attn)
 //   hy-worldplay/.../bi_sparse_operation_for_KV_cache.py:220-296 (generate_prefill_indices)
 #include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
@@ -448,6 +449,10 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> block_mask(const at::Tensor& q_po
                                        qs.data(), k_pool.data_ptr(), ks.data(), &p, indices.data_ptr<int32_t>(),
                                        counts.data_ptr<int32_t>(), return_scores ? scores.data_ptr() : nullptr,
                                        stream_of(q_pool)));
+  // The budgets are kept from an earlier call, which may have run on another
+  // stream: their memory is not to be handed out again before this launch ends.
+  if (p.row_budget)
+    row_budget->record_stream(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q_pool.device().index()).unwrap());
   return {indices, counts, scores};
 }
 

@@ -122,3 +122,34 @@ def test_two_streams_and_threads(dev):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert all(torch.equal(o.view(torch.int16), ref.view(torch.int16)) for v in outs.values() for o in v)
+
+
+@pytest.mark.parametrize("general", [False, True])
+def test_budgets_outlive_a_dropped_plan(dev, monkeypatch, general):
+    """The device copy of row budgets, made on one stream and read on another, is not handed out again while it is read."""
+    print(f"[gpu] row budgets of a dropped plan, general={general}", flush=True)
+    case = CASES[7]
+    x, params = _inputs(case, dev)
+    nq = _pipeline.geometry(case[5], (4, 8, 4), x[0].shape[2], x[3].shape[2], 0).nq_blk
+    params["row_budget"] = [(3 * i) % 5 + 1 for i in range(nq)]
+    if general:
+        monkeypatch.setattr(_pipeline, "native_call", lambda *a: None)
+    plans, masks = _pipeline._CALL_PLANS, _pipeline._core._MASK_PLANS
+    plans.clear()
+    masks.clear()
+    ref = _entry(case, x, params)
+    torch.cuda.synchronize()
+    (_, budgets), = masks.values()
+    at = budgets.data_ptr()
+    del budgets
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)   # a bounded wait, so that the call below is still to run
+        out = _entry(case, x, params)
+    plans.clear()
+    masks.clear()
+    taken = [torch.full((nq,), 7, dtype=torch.int32, device=dev) for _ in range(64)]
+    busy = not side.query()
+    torch.cuda.synchronize()
+    assert busy and all(t.data_ptr() != at for t in taken)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
