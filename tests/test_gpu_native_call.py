@@ -153,3 +153,28 @@ def test_budgets_outlive_a_dropped_plan(dev, monkeypatch, general):
     torch.cuda.synchronize()
     assert busy and all(t.data_ptr() != at for t in taken)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("case", [CASES[i] for i in (0, 3, 4, 6, 7, 8)])
+def test_captured_call_replays(dev, case):
+    """A call captured in a graph: every replay gives the bits of the eager call on the inputs that it finds."""
+    print(f"[gpu] captured call {case}", flush=True)
+    x, params = _inputs(case, dev)
+    if params.get("row_budget"):
+        nq = _pipeline.geometry(case[5], (4, 8, 4), x[0].shape[2], x[3].shape[2], 0).nq_blk
+        params["row_budget"] = [(3 * i) % 5 + 1 for i in range(nq)]
+    _entry(case, x, params)              # what is worked out once per configuration
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = _entry(case, x, params)
+    first = [t.clone() for t in x]
+    for i in range(4):
+        for t, f in zip(x, first):
+            t.copy_(f if i == 0 else f.roll(i, dims=2) * (1 - i / 8))
+        ref = _entry(case, x, params)
+        g.replay()
+        got = out.clone()
+        torch.cuda.synchronize()
+        assert torch.equal(got.contiguous().view(torch.int16), ref.contiguous().view(torch.int16)), i
+        torch.full((1 << 20,), float("nan"), device=dev)     # other work in the allocator's blocks between replays
