@@ -113,11 +113,12 @@ __device__ __forceinline__ void tile_unit(int& blk, int& bh) {
 // undo (heads along x), block coordinates take udiv16, all row loads of a batch
 // are unconditional (rows outside the grid read the block's first token, which
 // is always inside, and are replaced by zeros), a row's offset from the block's
-// first token takes 32 bits, and the job is read in one scalar round trip.Both pools of the 16-head 30 x 52 call with 4
-// + 12 frames (103 MB): 21.2 us, against 21.8 with a kernel of its own for the
-// pair and 24.1 with this one before those changes; the e4m3 tiles and pools of
-// the same call with 200 text tokens (156 MB): 31.8 us, against 43.2 in three
-// launches and 19 in four more for padding the text.
+// first token takes 32 bits, and the job is read in one scalar round trip.  Both
+// pools of the 16-head 30 x 52 call with 4 + 12 frames (103 MB): 21.2 us, against
+// 21.8 with a kernel of its own for the pair and 24.1 with this one before those
+// changes; the e4m3 tiles and pools of the same call with 200 text tokens (156
+// MB): 31.8 us, against 43.2 in three launches and 19 in four more for padding
+// the text.
 typedef __attribute__((address_space(4))) const PrepJob Job;
 
 template <typename E, int D, bool VEC>

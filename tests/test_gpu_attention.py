@@ -103,7 +103,8 @@ def split_per_xcd(tiles, cus):
 def test_tail_split_matches_whole_tiles_and_oracle(dev, H, nq):
     """Each XCD's tiles of a partial last round run as two halves of their block list plus a merge kernel
     when the round is at most half full (8 x 44 tiles on 256 CUs: 12 of each XCD's 44); a fuller last round
-    (8 x 58: 26 of 58) runs whole.  Both against whole tiles and the oracle."""
+    (8 x 58: 26 of 58) runs whole.  Both against whole tiles and the oracle.  li_bsa_fwd_workspace_size holds two halves
+    of each; lists as short as these are left whole all the same (test_gpu_split.py: 8 x 44 with lists that are not)."""
     from li_sparse import _lib
 
     bs, D, B, nkb = 128, 128, 1, 12

@@ -30,7 +30,7 @@ def _pieces(H, rows, cols, dev):
 
 # tiles below, at and above a multiple of 8 and of the CU count; lists shorter than, equal to and longer than the pieces
 @pytest.mark.parametrize("H,nq,cols", [(1, 1, 60), (1, 8, 40), (3, 5, 33), (1, 13, 21), (3, 17, 24), (2, 52, 40),
-                                       (5, 53, 16), (8, 33, 30)])
+                                       (5, 53, 16), (8, 33, 30), (8, 44, 24)])
 def test_pieces_match_whole_tiles_and_oracle(dev, H, nq, cols):
     bs, D, nkb = 128, 128, max(cols, 4) + 3
     Lq, Lk = nq * bs - 40, nkb * bs
