@@ -164,6 +164,11 @@ __device__ __forceinline__ void prep_block(Job& a, int b, int h, int blk) {
     bool ok[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) {
+      if constexpr (!VEC) {
+        ok[i] = false;
+        v[i] = u32x4{0u, 0u, 0u, 0u};
+        if (f0 + i * NG >= bs) continue;  // the whole workgroup
+      }
       const uint32_t f = f0 + i * NG + g0;
       const uint32_t r = udiv16(f, mg_tw), fw = f - r * tw;
       const uint32_t ft = udiv16(r, mg_th), fh = r - ft * th;
@@ -173,12 +178,20 @@ __device__ __forceinline__ void prep_block(Job& a, int b, int h, int blk) {
       // (checked on the host).
       if constexpr (VEC)
         v[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(sbase) + (l * (uint32_t)(2 * st_l) + 16u * c));
-      else
-        v[i] = load8(sbase + (int64_t)l * st_l + (int64_t)(8 * c) * st_d, st_d, vs);
+      else {
+        // A row at a time, and only rows that are there: with the element loads of
+        // eight rows in flight at once the kernel takes 226 VGPRs, and rows outside
+        // the block (three in four of a 64-row block at D = 64) would cost as much
+        // as the others.
+        if (ok[i]) v[i] = load8(sbase + (int64_t)l * st_l + (int64_t)(8 * c) * st_d, st_d, vs);
+        asm volatile("" : "+v"(v[i])::"memory");
+      }
     }
+    if constexpr (VEC) {
 #pragma unroll
-    for (int i = 0; i < R; ++i)
-      if (!ok[i]) v[i] = u32x4{0u, 0u, 0u, 0u};
+      for (int i = 0; i < R; ++i)
+        if (!ok[i]) v[i] = u32x4{0u, 0u, 0u, 0u};
+    }
     if (dst) {
       const int64_t doff = b * a.ds[0] + h * a.ds[1] + (blk + a.dst_off) * a.ds[2];
       if (scale) {
