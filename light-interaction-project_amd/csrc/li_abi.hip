@@ -1,6 +1,8 @@
 // Version, status strings and the last launch error of the sparse-attention C ABI.
 #include <stdio.h>
 
+#include <mutex>
+
 #include "li_common.hpp"
 
 namespace {
@@ -9,6 +11,20 @@ thread_local char g_last_error[256] = "no launch error";
 
 void li::record_launch_error(hipError_t e) {
   snprintf(g_last_error, sizeof(g_last_error), "%s: %s", hipGetErrorName(e), hipGetErrorString(e));
+}
+
+int li::device_cus() {
+  static std::mutex mu;
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  std::lock_guard<std::mutex> lock(mu);
+  if (cached[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
+    cached[dev] = n > 0 ? n : -1;
+  }
+  return cached[dev] > 0 ? cached[dev] : 0;
 }
 
 extern "C" const char* li_last_error(void) { return g_last_error; }

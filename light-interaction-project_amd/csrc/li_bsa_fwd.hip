@@ -1634,21 +1634,6 @@ __global__ __launch_bounds__(256) void bsa_merge_kernel(BsaArgs a) {
   if (a.lse && dq == 0) a.lse[(int64_t)bh * a.Lq + r] = mm == -__builtin_inff() ? mm : mm + __builtin_log2f(l);
 }
 
-// Compute units of the current device, cached per device.
-int device_cus() {
-  static std::mutex mu;
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  std::lock_guard<std::mutex> lock(mu);
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
-    cached[dev] = n > 0 ? n : -1;
-  }
-  return cached[dev] > 0 ? cached[dev] : 0;
-}
-
 // Workgroups of an attention launch: the tiles, or per XCD its whole tiles and
 // the pieces of at most xsplit split ones.
 int attn_units(const BsaArgs& a) { return a.xparts == 0 ? a.ntiles : 8 * (a.xwhole + a.xsplit * a.xparts); }
@@ -1713,8 +1698,11 @@ int launch_bsa_d64(BsaArgs& a, hipStream_t s) {
   clear_launch_error();
   // With a tile per CU at most, eight waves and four interleaves per tile; with
   // more, four waves and two, so that two workgroups share a CU and one's loads
-  // and barriers hide behind the other's work.
-  if (a.ntiles <= device_cus())
+  // and barriers hide behind the other's work.  Lists of up to ten blocks take two
+  // as well: the merge of four costs more than their steps save (us at 4 x 64 tiles
+  // of 1, 4, 8, 10, 12 and 16 blocks: 6.3, 7.4, 8.6, 9.4, 9.9 and 11.0 with four, 5.6,
+  // 6.7, 8.5, 9.3, 10.1 and 11.8 with two).
+  if (a.ntiles <= device_cus() && a.n_cols > 10)
     hipLaunchKernelGGL((bsa_fwd_d64_kernel<E, QO, 4>), dim3(a.ntiles), dim3(512), 0, s, a);
   else
     hipLaunchKernelGGL((bsa_fwd_d64_kernel<E, QO, 2>), dim3(a.ntiles), dim3(256), 0, s, a);

@@ -96,4 +96,7 @@ inline int launch_status() {
   return LI_ERR_LAUNCH;
 }
 
+// Compute units of the current device (cached per device), or 0.
+int device_cus();
+
 }  // namespace li

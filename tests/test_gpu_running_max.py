@@ -84,6 +84,7 @@ def test_blocks_far_above_the_running_max(dev, kind, D, bs, H, nq, dtype):
         for at, many in (((1,), False), ((4, 7), False), ((5,), True), ((8,), False)):
             q, k, v, scale = _case(D, bs, H, nq, dtype, jump, at, many, gen)
             ind = torch.arange(COLS, dtype=torch.int32).repeat(1, H, nq, 1)
+            ind = torch.nn.functional.pad(ind, (0, 3), value=-1)   # wide enough for four interleaves; never read
             cnt = torch.full((1, H, nq), COLS, dtype=torch.int32)
             if kind != "dense":  # shorter lists too: the raised block the last one, or absent
                 cnt[0, 0] = torch.from_numpy(rng.integers(at[0], COLS + 1, nq).astype(np.int32))
