@@ -257,13 +257,12 @@ struct RowGeom {
   }
 };
 
-// Step 1b/2 for one (row, block): score bits from the fp32 dot product, the
+// Step 1b/2 for one (row, block): score bits from the dot product in E, the
 // forced flag, and the order key (0 for a forced block).  mg_hw, mg_nw: udiv16
 // magics of the key grid's slab and row (nk <= kMaxNk < 2^16).
 template <typename E>
 __device__ __forceinline__ uint32_t finish_key(const li_mask_params& p, const RowGeom& g, uint16_t* srow, int j,
-                                               float dot, bool& f, uint32_t mg_hw, uint32_t mg_nw) {
-  uint16_t s = E::from_f32(dot);
+                                               uint16_t s, bool& f, uint32_t mg_hw, uint32_t mg_nw) {
   if (p.metric == LI_METRIC_SCALED_DOT) s = E::from_f32(E::to_f32(s) * p.scale);
   if (srow) srow[j] = s;
   f = (p.n_recent > 0) && (j >= g.nk - p.n_recent);
@@ -315,8 +314,7 @@ __global__ __launch_bounds__(256) void block_mask_kernel(MaskArgs a, int waves) 
 #pragma unroll
         for (int d = 0; d < D; ++d) ps[d & 7] = ps[d & 7] + qv[d] * x[d];
       }
-      const float dot = sum8(ps);
-      keys[j] = finish_key<E>(p, g, srow, j, dot, f, a.mg_hw, a.mg_nw);
+      keys[j] = finish_key<E>(p, g, srow, j, E::from_f32(sum8(ps)), f, a.mg_hw, a.mg_nw);
     }
     nf += wave_count(f);
   }
@@ -346,6 +344,9 @@ __global__ __launch_bounds__(256) void block_mask_kernel(MaskArgs a, int waves) 
 // workgroup with two waves per row on the vector ALU (rows x blocks):
 //   896 x 168  10.3 -> 9.9    1248 x 104 (cosine) 15.3 -> 11.4   256 x 64 (D = 64) 6.3 -> 6.1
 //   2496 x 156 24.0 -> 16.6    720 x 150 (cosine) 11.7 -> 10.5   896 x 896 27.6 -> 25.6
+// The scores wait for their selection in 16 bits (the type that they are rounded
+// to first thing), which with SW = 4 leaves LDS for two workgroups a CU up to
+// 1024 blocks; see li_block_mask for the choice of SW.
 template <typename E, int D, int KS, int SW>
 __global__ __launch_bounds__(512) void block_mask_rows_kernel(MaskArgs a) {
   constexpr int CH = D / 8;           // 16-byte granules per pool row
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(512) void block_mask_rows_kernel(MaskArgs a) {
   typedef __attribute__((address_space(3))) void lds_void;
   __shared__ __attribute__((aligned(16))) char stage[SW][64 * RB];
   __shared__ __attribute__((aligned(16))) float qall[4][QP];
-  __shared__ __attribute__((aligned(16))) float dots[4][64 * KS];
+  __shared__ __attribute__((aligned(16))) uint16_t dots[4][64 * KS];
   const li_mask_params& p = a.p;
   const int nk = p.nk, nchunk = (nk + 63) / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -445,13 +446,14 @@ __global__ __launch_bounds__(512) void block_mask_rows_kernel(MaskArgs a) {
     }
     // Every read of the stage has completed (its values went into the products).
     if (chunk + SW < nchunk) stage_chunk(chunk + SW);
-    f32x4 dot;
+    uint16_t dot[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float s8[8] = {ps[0][r], ps[1][r], ps[2][r], ps[3][r], ps[4][r], ps[5][r], ps[6][r], ps[7][r]};
-      dot[r] = sum8(s8);
+      dot[r] = E::from_f32(sum8(s8));
     }
-    *reinterpret_cast<f32x4*>(&dots[lane & 3][64 * chunk + 4 * (lane >> 2)]) = dot;
+    *reinterpret_cast<u32x2*>(&dots[lane & 3][64 * chunk + 4 * (lane >> 2)]) =
+        u32x2{pack2(dot[0], dot[1]), pack2(dot[2], dot[3])};
   }
   __syncthreads();
   const int qb = qb0 + wave;
@@ -557,10 +559,22 @@ extern "C" int li_block_mask(int dtype, int32_t B, int32_t NH, int32_t D, const 
   if (shared) grid = dim3((unsigned)(a.groups * a.NBH));
   hipStream_t s = static_cast<hipStream_t>(stream);
   clear_launch_error();
+  // Past 256 blocks eight scoring waves end a workgroup soonest, but hold a CU's
+  // LDS (D = 128); once the row groups outnumber the CUs, four of them and two
+  // workgroups a CU are faster.  Kernel times, us, SW = 8 and 4 (heads x rows x
+  // blocks, scaled dot product):
+  //   16 x 56 x 896 (224 groups)  18.7, 20.3     16 x 72 x 300 (288)   23.5, 16.2
+  //    1 x 1000 x 1000 (250)      19.3, 20.8     16 x 156 x 600 (624)  44.0, 32.0
+  //   16 x 64 x 300 (256)         14.1, 14.9     16 x 1000 x 512       194.2, 113.6
+  // and D = 64, 8 x 300 x 300: 21.0, 17.3.  Past 1024 blocks SW = 4 does not fit twice
+  // either (16 x 300 x 1500: 128.7, 141.0).
+  const bool many = (int64_t)a.groups * a.NBH > device_cus();
 #define LI_MASK_LAUNCH(E_, D_)                                                                           \
   do {                                                                                                   \
     if (shared && p.nk <= 256)                                                                           \
       hipLaunchKernelGGL((block_mask_rows_kernel<E_, D_, 4, 4>), grid, dim3(512), lds, s, a);            \
+    else if (shared && p.nk <= 1024 && many)                                                             \
+      hipLaunchKernelGGL((block_mask_rows_kernel<E_, D_, 16, 4>), grid, dim3(512), lds, s, a);           \
     else if (shared && p.nk <= 1024)                                                                     \
       hipLaunchKernelGGL((block_mask_rows_kernel<E_, D_, 16, 8>), grid, dim3(512), lds, s, a);           \
     else if (shared)                                                                                     \

@@ -37,6 +37,24 @@ def test_equals_generic_kernel(dev, nk, D, dtype):
                                    y.view(torch.int16) if y.dtype != torch.int32 else y), (nq, metric, kw)
 
 
+@pytest.mark.parametrize("nk", [257, 320, 700, 1024])
+@pytest.mark.parametrize("D,dtype", [(128, torch.float16), (64, torch.bfloat16)])
+def test_many_row_groups_equal_generic_kernel(dev, nk, D, dtype):
+    """More row groups than CUs: four scoring waves a workgroup."""
+    NH, nq = 8, 4 * (torch.cuda.get_device_properties(dev).multi_processor_count // 8) + 3
+    print(f"[gpu] block mask, many rows: {NH} x {nq} x {nk} D={D} {dtype}", flush=True)
+    q, k = _pools(1, NH, nq, nk, D, dtype, dev, nk)
+    strided = torch.stack([k, k], -1)[..., 0]
+    for metric in ("cosine", "scaled_dot_product"):
+        kw = dict(metric=metric, nh=3, nw=7, num_txt_blk=1, return_scores=True, budget_mode=_lib.LI_BUDGET_HISTORY,
+                  ratio=0.3, n_recent=2, force_diag=True)
+        a, b = _core.block_mask(q, k, **kw), _core.block_mask(q, strided, **kw)
+        torch.cuda.synchronize()
+        for x, y in zip(a, b):
+            assert torch.equal(x.view(torch.int16) if x.dtype != torch.int32 else x,
+                               y.view(torch.int16) if y.dtype != torch.int32 else y), metric
+
+
 def test_special_values_and_strided_pools(dev):
     """Infinities, NaN and the smallest numbers in the pools; pools that are views of longer buffers."""
     B, NH, nq, nk, D = 2, 2, 6, 130, 128
