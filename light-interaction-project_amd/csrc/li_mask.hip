@@ -357,6 +357,9 @@ __global__ __launch_bounds__(512) void block_mask_rows_kernel(MaskArgs a) {
   __shared__ __attribute__((aligned(16))) char stage[SW][64 * RB];
   __shared__ __attribute__((aligned(16))) float qall[4][QP];
   __shared__ __attribute__((aligned(16))) uint16_t dots[4][64 * KS];
+  // With a chunk per scoring wave at most, all waves share the raw pool's divisions.
+  constexpr bool kShareDiv = KS <= SW;
+  __shared__ float dens[kShareDiv ? 64 * KS : 1];
   const li_mask_params& p = a.p;
   const int nk = p.nk, nchunk = (nk + 63) / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -397,38 +400,56 @@ __global__ __launch_bounds__(512) void block_mask_rows_kernel(MaskArgs a) {
   wait_vm0();
   __syncthreads();
 
+  // Normaliser of this lane's block in the wave's stage, and the division of a
+  // granule of a raw pool row by its normaliser.
+  auto normaliser = [&]() LI_MASK_INLINE {
+    float ss = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const u32x4 w = *reinterpret_cast<const u32x4*>(st + lane * RB + 16 * (c ^ swz(lane)));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float x = E::to_f32(uint16_t((w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu));
+        ss = ss + x * x;
+      }
+    }
+    const float nrm = E::to_f32(E::from_f32(__builtin_sqrtf(ss)));
+    const float eps = E::to_f32(E::from_f32(1e-12f));
+    return nrm > eps ? nrm : eps;
+  };
+  auto divide = [&](char* at, float den) LI_MASK_INLINE {
+    u32x4 w = *reinterpret_cast<u32x4*>(at);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t lo = E::from_f32(E::to_f32(uint16_t(w[e] & 0xFFFFu)) / den);
+      const uint32_t hi = E::from_f32(E::to_f32(uint16_t(w[e] >> 16)) / den);
+      w[e] = lo | (hi << 16);
+    }
+    *reinterpret_cast<u32x4*>(at) = w;
+  };
+  const bool raw_cosine = cosine && !p.k_normalized;
+  if constexpr (kShareDiv) {
+    if (raw_cosine) {
+      if (scores && sw < nchunk) dens[64 * sw + lane] = normaliser();
+      __syncthreads();
+      // Granules of the rows that are there, eight divisions each: the longest part
+      // of a small raw cosine call when a lane does its whole row (1 x 4 x 16 blocks,
+      // D = 64: 6.8 us).
+      for (int i = tid; i < nk * CH; i += 512) divide(stage[i / (64 * CH)] + (i % (64 * CH)) * 16, dens[i / CH]);
+      __syncthreads();
+    }
+  }
+
   // Lane l of a 4x4x1 product: A = block l, B = query row l % 4; its result
   // element r is block 4 (l / 4) + r for query row l % 4.
   const float* qrow = qall[lane & 3];
   for (int chunk = scores ? sw : nchunk; chunk < nchunk; chunk += SW) {
     if (chunk != sw) wait_vm0();
-    if (cosine && !p.k_normalized) {
+    if (!kShareDiv && raw_cosine) {
       // The raw pool's rows, normalised in place by their lanes.
-      float ss = 0.0f;
+      const float den = normaliser();
 #pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(st + lane * RB + 16 * (c ^ swz(lane)));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float x = E::to_f32(uint16_t((w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu));
-          ss = ss + x * x;
-        }
-      }
-      const float nrm = E::to_f32(E::from_f32(__builtin_sqrtf(ss)));
-      const float eps = E::to_f32(E::from_f32(1e-12f));
-      const float den = nrm > eps ? nrm : eps;
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        u32x4* at = reinterpret_cast<u32x4*>(st + lane * RB + 16 * (c ^ swz(lane)));
-        u32x4 w = *at;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t lo = E::from_f32(E::to_f32(uint16_t(w[e] & 0xFFFFu)) / den);
-          const uint32_t hi = E::from_f32(E::to_f32(uint16_t(w[e] >> 16)) / den);
-          w[e] = lo | (hi << 16);
-        }
-        *at = w;
-      }
+      for (int c = 0; c < CH; ++c) divide(st + lane * RB + 16 * (c ^ swz(lane)), den);
     }
     f32x4 ps[8];
 #pragma unroll
