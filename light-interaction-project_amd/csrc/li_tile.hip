@@ -182,7 +182,8 @@ __device__ __forceinline__ void prep_block(Job& a, int b, int h, int blk) {
         // A row at a time, and only rows that are there: with the element loads of
         // eight rows in flight at once the kernel takes 226 VGPRs, and rows outside
         // the block (three in four of a 64-row block at D = 64) would cost as much
-        // as the others.
+        // as the others: tiles and pool of 16 heads x 12 frames x 30 x 52 97.1 us
+        // that way, 78.2 this way; K and V of 8 heads x 2 x 32 x 32 at D = 64 23.2, 8.3.
         if (ok[i]) v[i] = load8(sbase + (int64_t)l * st_l + (int64_t)(8 * c) * st_d, st_d, vs);
         asm volatile("" : "+v"(v[i])::"memory");
       }
