@@ -1800,20 +1800,21 @@ double units_us(int64_t n, double blocks, int64_t c) {
 //
 // The constants were fitted to the choice, not to the times: over 225 sizes (8
 // to 1500 tiles of 8 to 80 blocks), each run whole and with 2 to 16 pieces in bf16
-// and in e4m3, the chosen number is within 0.2% of the best one in the mean (7% at
-// worst), and at most 1% (one e4m3 size 3%) slower than two pieces behind a last
-// round at most half full and whole tiles otherwise.  One merge price for both
+// and in e4m3, the chosen number is within 0.2% of the best one in the mean (10% at
+// worst), and at most 1% slower than two pieces behind a last round at most half
+// full and whole tiles otherwise.  One merge price for both
 // kinds of launch lost 1 to 9% to that at lists of 12 to 36 blocks behind a last
 // round about half full, and 5% with pieces of short lists in a small launch.
 // Attention and merge, us (tiles x blocks; f16 as bf16):
-//     8 x 60  bf16:  66.6, 10 pieces 20.1       52 x 16  bf16: 23.9, 2 pieces 22.6, 4 pieces 23.4
-//   104 x 40  bf16:  51.2,  2 pieces 41.8       52 x 16  e4m3: 21.9, 2 pieces 20.7, 4 pieces 23.1
+//     8 x 60  bf16:  66.6, 10 pieces 20.1       52 x 24  bf16: 32.4, 3 pieces 24.3
+//   104 x 40  bf16:  51.2,  2 pieces 41.8       52 x 24  e4m3: 29.5, 3 pieces 23.1
 //   352 x 24  bf16:  81.9,  2 pieces 76.4      352 x 24  e4m3: 70.9, 2 pieces 65.3
 //   384 x 36  bf16: 117.1,  2 pieces 110.3     384 x 36  e4m3: 101.7, 2 pieces 92.9
 //   784 x 50  bf16: 320.9, 10 pieces 285.7     896 x 36  e4m3: 207.7, 2 pieces 198.9
 //   896 x 51  bf16: 329.6,  2 pieces 324.4     896 x 36  bf16: 245.5, 2 pieces 238.6
 // and whole tiles stay the better ones at 104 x 16 (25.5 against 29.7), 52 x 8 (16.3,
-// 18.7), 160 x 40 (59.6, 66.2) and 472 x 36 (125.5, 140.8).
+// 18.7), 160 x 40 (59.6, 66.2) and 472 x 36 (125.5, 140.8); 52 x 16 (23.9, 22.6) is left
+// whole for the launch.
 SplitPlan plan_split(int64_t tiles, int64_t n_cols, int cus, int64_t bytes) {
   SplitPlan best;
   if (cus <= 0 || cus % 8 != 0 || n_cols <= 0) return best;
@@ -1821,7 +1822,9 @@ SplitPlan plan_split(int64_t tiles, int64_t n_cols, int cus, int64_t bytes) {
   if (r == 0) return best;
   const double merge = n < c ? 1.0 : 3.0, merge_piece = n < c ? 0.046 : 0.019;
   const int64_t most = (bytes < kMaxPartBytes ? bytes : kMaxPartBytes) / (8 * kPartBytes);  // pieces per XCD
-  double cost = units_us(r, (double)n_cols, c) - 1.0;  // a gain of less than 1 us is left
+  // A gain of less than 1 us is left, and one of less than 3 us in a launch of one
+  // round: such calls wait on the host, and the merge is a launch more (2.5 us).
+  double cost = units_us(r, (double)n_cols, c) - (n < c ? 3.0 : 1.0);
   for (int64_t parts = 2; parts * r <= most && parts <= n_cols; ++parts) {
     const double blocks = (double)((n_cols + parts - 1) / parts);
     const double t = units_us(r * parts, blocks, c) + merge + merge_piece * 8.0 * (double)(r * parts);

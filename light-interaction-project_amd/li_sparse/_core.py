@@ -214,7 +214,7 @@ def prep(q, q_pool, geom_q, k, v, k_pool, first, geom_k, *, q_tiles=None, q_scal
     if v_tiles is not None and tuple(v.shape) != tuple(k.shape):
         raise ValueError(f"K/V source shapes differ: {tuple(k.shape)} vs {tuple(v.shape)}")
     k_txt, v_txt = text if text is not None else (None, None)
-    _run(ops.prep, q, q_tiles, q_scale, q_pool, geom_q, k, v, k_tiles, k_scale, v_tiles, k_pool, k_pool_n, first, geom_k,
+    _run(ops.prep.default, q, q_tiles, q_scale, q_pool, geom_q, k, v, k_tiles, k_scale, v_tiles, k_pool, k_pool_n, first, geom_k,
          num_txt_blk, k_txt, v_txt, *padded_text)
 
 

@@ -363,8 +363,10 @@ def native_call(mode, q, k_txt, v_txt, k_vis, v_vis, latent_hw, tile, p, default
     """The whole call as one operator (``li::sparse_call``: the launches of ``sparse_attention``, with the host work
     between them in C++), or None for what it leaves to ``sparse_attention``: a context cache, element types and
     shapes that have to be converted or refused there, parameters that cannot be looked up."""
+    if p.get("context_cache") is not None:
+        return None
     dt, dev, shape = q.dtype, q.device, q.shape
-    if (dt is not torch.bfloat16 and dt is not torch.float16) or dev.type != "cuda" or p.get("context_cache") is not None:
+    if (dt is not torch.bfloat16 and dt is not torch.float16) or dev.type != "cuda":
         return None
     if p.get("qk_fp8") and dt is not torch.bfloat16:
         return None
