@@ -1972,8 +1972,12 @@ bool row_view_ok(const void* p, const int64_t st[4]) {
 // 32 MiB reaches the largest row offset of the call shapes of both models
 // (HY-WorldPlay's (4, 8, 4) tile over a 30 x 52 grid: 5047 tokens of up to
 // 24 heads x 128 bf16 = 31 MB); larger calls pick their sources per chunk.
+// On a page boundary: at the 256-byte one where the code before it happened to
+// end, calls with much padding or text ran 0.5 to 1.5% slower or not with every
+// change of the code's size (12 heads, 43 x 64 grid, 12 text tokens: 934.4 us at
+// offset 0x100, 928.5 at 0; 7 heads, 51 x 88, ragged: 803.5 at 0x700, 793.8).
 constexpr int64_t kZeroRegionBytes = 32ll << 20;
-static __device__ __align__(256) char g_zero_region[kZeroRegionBytes];
+static __device__ __align__(4096) char g_zero_region[kZeroRegionBytes];
 
 namespace {
 
