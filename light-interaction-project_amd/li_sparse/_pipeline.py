@@ -325,28 +325,32 @@ def _call_plan(mode, dev, lq, lk, text_len, D, latent_hw, tile, p, default_ratio
     A configuration is looked up by the values that its parameters resolve to, read anew for each call: an absent key
     and an explicit None are not the same for all of them, and a parameter may be an object that changes in place.
     """
-    (H, W), (tt, th, tw) = latent_hw, tile
-    latent_hw, tile = (index(H), index(W)), (index(tt), index(th), index(tw))
-    fp8, decode = qk_fp8(p), mode == "decode"
-    if fp8 and not fp8_supported(D, tile):
+    H, W = latent_hw
+    tt, th, tw = tile
+    if not (H.__class__ is W.__class__ is tt.__class__ is th.__class__ is tw.__class__ is int):
+        H, W, tt, th, tw = index(H), index(W), index(tt), index(th), index(tw)
+    get, decode = p.get, mode == "decode"
+    fp8 = bool(get("qk_fp8", False))
+    if fp8 and not fp8_supported(D, (tt, th, tw)):
         return None
-    rb, rb_key = p.get("row_budget"), None
+    rb, rb_key = get("row_budget"), None
     if rb is not None:
         rb = np.asarray(rb) if isinstance(rb, (list, tuple, np.ndarray)) else None
         if rb is None or rb.ndim != 1 or rb.dtype.kind not in "iub":
             return None
         rb_key = (rb.dtype.str, rb.tobytes())
-    protect = p.get("recent_protect", 0) if decode else 0
-    if not isinstance(protect, Real):
+    protect = get("recent_protect", 0) if decode else 0
+    if protect.__class__ is not int and not isinstance(protect, Real):
         return None
-    diag, sink = bool(p.get("force_diag", False)), bool(p.get("force_sink", False))
-    ratio = float(p.get("topk_ratio", 1.0 if decode else default_ratio))
-    metric, cos = _core.METRICS.get(p.get("sim_metric", "cosine"), _lib.LI_METRIC_DOT), cosine(p)
-    key = (decode, dev, lq, lk, text_len, D, latent_hw, tile, ratio, metric, cos, protect, diag, sink, fp8, rb_key)
+    diag, sink = bool(get("force_diag", False)), bool(get("force_sink", False))
+    ratio = float(get("topk_ratio", 1.0 if decode else default_ratio))
+    sim = get("sim_metric", "cosine")
+    metric, cos = _core.METRICS.get(sim, _lib.LI_METRIC_DOT), sim == "cosine"
+    key = (decode, dev, lq, lk, text_len, D, H, W, tt, th, tw, ratio, metric, cos, protect, diag, sink, fp8, rb_key)
     plan = _CALL_PLANS.get(key)
     if plan is not None:
         return plan
-    g = geometry(latent_hw, tile, lq, lk, text_len)
+    g = geometry((H, W), (tt, th, tw), lq, lk, text_len)
     n_recent = recent_blocks(p, g.tt, g.nh, g.nw, g.nk_blk) if decode else 0
     budget = _lib.LI_BUDGET_HISTORY if decode else _lib.LI_BUDGET_TOTAL
     kmax, rb_dev = _core._mask_plan(dev, g.nq_blk, g.nk_blk, g.nh, g.nw, g.num_txt_blk, n_recent, diag, sink, not decode,
