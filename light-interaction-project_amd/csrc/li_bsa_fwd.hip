@@ -1813,8 +1813,7 @@ double units_us(int64_t n, double blocks, int64_t c) {
 //   784 x 50  bf16: 320.9, 10 pieces 285.7     896 x 36  e4m3: 207.7, 2 pieces 198.9
 //   896 x 51  bf16: 329.6,  2 pieces 324.4     896 x 36  bf16: 245.5, 2 pieces 238.6
 // and whole tiles stay the better ones at 104 x 16 (25.5 against 29.7), 52 x 8 (16.3,
-// 18.7), 160 x 40 (59.6, 66.2) and 472 x 36 (125.5, 140.8); 52 x 16 (23.9, 22.6) is left
-// whole for the launch.
+// 18.7), 160 x 40 (59.6, 66.2) and 472 x 36 (125.5, 140.8).
 SplitPlan plan_split(int64_t tiles, int64_t n_cols, int cus, int64_t bytes) {
   SplitPlan best;
   if (cus <= 0 || cus % 8 != 0 || n_cols <= 0) return best;
@@ -1822,9 +1821,11 @@ SplitPlan plan_split(int64_t tiles, int64_t n_cols, int cus, int64_t bytes) {
   if (r == 0) return best;
   const double merge = n < c ? 1.0 : 3.0, merge_piece = n < c ? 0.046 : 0.019;
   const int64_t most = (bytes < kMaxPartBytes ? bytes : kMaxPartBytes) / (8 * kPartBytes);  // pieces per XCD
-  // A gain of less than 1 us is left, and one of less than 3 us in a launch of one
-  // round: such calls wait on the host, and the merge is a launch more (2.5 us).
-  double cost = units_us(r, (double)n_cols, c) - (n < c ? 3.0 : 1.0);
+  // A gain of less than 1 us is left, and one of less than 2 us in a launch of one
+  // round: where such a call waits on the host, the merge's launch costs it 2.5 us
+  // (a cached call with 28 tiles of 10 blocks: 52.3 us, whole 49.9; a dense one, which
+  // does not wait, with 56 tiles of 16: 32.3 whole, 29.5 in two pieces).
+  double cost = units_us(r, (double)n_cols, c) - (n < c ? 2.0 : 1.0);
   for (int64_t parts = 2; parts * r <= most && parts <= n_cols; ++parts) {
     const double blocks = (double)((n_cols + parts - 1) / parts);
     const double t = units_us(r * parts, blocks, c) + merge + merge_piece * 8.0 * (double)(r * parts);
